@@ -30,31 +30,43 @@ constexpr int kHeadParams = kCh + 1 + kHid * kP + kHid + kHid + 1;
 inline int conv_cin(int layer) { return layer == 0 ? 32 : kCh; }
 inline int conv_weights(int layer) { return kCh * conv_cin(layer) * 9; }
 
-// Packed MFMA A-operand weights of one conv, forward or (64 -> 64 only)
-// backward-data (transposed, taps flipped): 9 * cin * 64 BF16 values.
-hipError_t pack_conv(const float *w, uint16_t *wpk, int cin, bool bwd,
-                     hipStream_t stream);
+// Packed MFMA A-operand weights (BF16, 9 * cin * 64 values a conv) of every
+// conv from its FP32 weights w: forward (wf) and, from conv 1 on,
+// backward-data (wb: transposed, taps flipped).
+struct PackArgs {
+    const float *w[kNConv];
+    uint16_t *wf[kNConv], *wb[kNConv];
+};
+hipError_t pack(const PackArgs &a, hipStream_t stream);
 
-// One conv over n boards. Forward (bwd = false): out = elu(conv(in) + bias
-// + res). Backward-data (bwd = true, cin 64): out = (conv(in) + res) masked
-// where mask > 0. res and mask may be null. in is u8 planes [n][32][361]
-// when cin == 32, else BF16 [n][361][64].
-hipError_t conv(const void *in, int cin, const uint16_t *wpk,
-                const float *bias, const uint16_t *res, const uint16_t *mask,
-                uint16_t *out, int n, bool bwd, hipStream_t stream);
+// The network's forward pass over n boards (planes u8 [n][32][361]): conv
+// l's output to act + l * map_elems (BF16 [n][361][64]), the head's s
+// [n][361], f [n][64] and t [n] (the backward pass reads them), win [n] =
+// (1 + t) / 2 (may be null). w: packed forward weights, b: biases, hp: the
+// head parameters. train: a backward pass follows and reads the maps.
+struct FwdArgs {
+    const uint16_t *w[kNConv];
+    const float *b[kNConv];
+};
+hipError_t forward(const uint8_t *planes, const FwdArgs &a, uint16_t *act,
+                   size_t map_elems, const float *hp, float *s, float *f,
+                   float *t, float *win, int n, bool train,
+                   hipStream_t stream);
+
+// Backward-data of one 64 -> 64 conv over n boards: out = (conv(e) + res)
+// times ELU's derivative at the activation mask. res may be null. Maps BF16
+// [n][361][64].
+hipError_t conv_bwd(const uint16_t *e, const uint16_t *wpk,
+                    const uint16_t *res, const uint16_t *mask, uint16_t *out,
+                    int n, hipStream_t stream);
 
 // Weight and bias gradient of one conv: gW (OIHW) and gb are written (not
 // accumulated). e: BF16 [n][361][64] gradient at the conv's pre-activation;
-// in: the conv's input as for conv(). part must hold
+// in: the conv's input (u8 planes when cin == 32). part must hold
 // wgrad_part_floats(cin, n) floats.
 size_t wgrad_part_floats(int cin, int n);
 hipError_t wgrad(const void *in, int cin, const uint16_t *e, float *part,
                  float *gW, float *gb, int n, hipStream_t stream);
-
-// Head forward: s [n][361], f [n][64], t [n] kept for the backward pass;
-// win [n] = (1 + t) / 2 (may be null).
-hipError_t head_fwd(const uint16_t *h, const float *hp, float *s, float *f,
-                    float *t, float *win, int n, hipStream_t stream);
 
 // Loss mean_n (t - (2y - 1))^2, head gradients (into ghp, written), the
 // BF16 gradient e [n][361][64] at the last conv's pre-activation, and the

@@ -111,37 +111,34 @@ void release(lz_surrogate *s) {
 
 int repack(lz_surrogate *s, hipStream_t st) {
     const Layout &L = layout();
+    PackArgs a = {};
     for (int l = 0; l < kNConv; l++) {
-        int rc = s->hip(pack_conv(s->p + L.w[l], s->wf[l], conv_cin(l), false,
-                                  st), "pack");
-        if (rc) return rc;
-        if (l > 0) {
-            rc = s->hip(pack_conv(s->p + L.w[l], s->wb[l], kCh, true, st),
-                        "pack");
-            if (rc) return rc;
-        }
+        a.w[l] = s->p + L.w[l];
+        a.wf[l] = s->wf[l];
+        a.wb[l] = s->wb[l];
     }
-    s->packed = true;
-    return LZ_OK;
+    int rc = s->hip(pack(a, st), "pack");
+    if (!rc) s->packed = true;
+    return rc;
 }
 
-// Forward over n boards of device planes; keeps every activation.
+// Forward over n boards of device planes; keeps every activation. train: a
+// backward pass follows.
 int forward(lz_surrogate *s, int n, const uint8_t *planes, float *win,
-            hipStream_t st) {
+            bool train, hipStream_t st) {
     const Layout &L = layout();
     if (!s->packed) {
         int rc = repack(s, st);
         if (rc) return rc;
     }
+    FwdArgs a = {};
     for (int l = 0; l < kNConv; l++) {
-        const void *in = l == 0 ? (const void *)planes : (const void *)s->act_of(l - 1);
-        const uint16_t *res = (l >= 2 && l % 2 == 0) ? s->act_of(l - 2) : nullptr;
-        int rc = s->hip(conv(in, conv_cin(l), s->wf[l], s->p + L.b[l], res,
-                             nullptr, s->act_of(l), n, false, st), "conv");
-        if (rc) return rc;
+        a.w[l] = s->wf[l];
+        a.b[l] = s->p + L.b[l];
     }
-    return s->hip(head_fwd(s->act_of(kNConv - 1), s->p + L.head, s->s, s->f,
-                           s->t, win, n, st), "head_fwd");
+    return s->hip(lz::sg::forward(planes, a, s->act, s->map_elems(),
+                                  s->p + L.head, s->s, s->f, s->t, win, n,
+                                  train, st), "forward");
 }
 
 // Backward of the last forward into s->g (written, not accumulated); the
@@ -161,9 +158,8 @@ int backward(lz_surrogate *s, int n, const uint8_t *planes, const float *y,
                           s->g + L.w[l], s->g + L.b[l], n, st), "wgrad");
         if (rc) return rc;
         const uint16_t *res = (l % 2 == 1) ? s->emap(l + 1) : nullptr;
-        rc = s->hip(conv(s->emap(l), kCh, s->wb[l], nullptr, res,
-                         s->act_of(l - 1), s->emap(l - 1), n, true, st),
-                    "conv_bwd");
+        rc = s->hip(conv_bwd(s->emap(l), s->wb[l], res, s->act_of(l - 1),
+                             s->emap(l - 1), n, st), "conv_bwd");
     }
     if (rc) return rc;
     return s->hip(wgrad(planes, 32, s->emap(0), s->part, s->g + L.w[0],
@@ -321,7 +317,7 @@ int lz_surrogate_forward_device(lz_surrogate *s, int n, const uint8_t *planes,
     std::lock_guard<std::mutex> g(s->mu);
     hipStream_t st = (hipStream_t)stream;  // NULL: the default stream
     rc = join(s, s->stream, st);
-    if (!rc) rc = forward(s, n, planes, winrate, st);
+    if (!rc) rc = forward(s, n, planes, winrate, false, st);
     if (!rc) rc = join(s, st, s->stream);
     return rc;
 }
@@ -334,7 +330,7 @@ int lz_surrogate_predict(lz_surrogate *s, int n, const uint8_t *planes,
     std::lock_guard<std::mutex> g(s->mu);
     rc = s->hip(hipMemcpyAsync(s->planes, planes, (size_t)n * 32 * kP,
                                hipMemcpyHostToDevice, s->stream), "copy planes");
-    if (!rc) rc = forward(s, n, s->planes, s->win, s->stream);
+    if (!rc) rc = forward(s, n, s->planes, s->win, false, s->stream);
     if (!rc) rc = s->hip(hipMemcpyAsync(winrate, s->win, n * sizeof(float),
                                         hipMemcpyDeviceToHost, s->stream), "copy out");
     if (!rc) rc = s->hip(hipStreamSynchronize(s->stream), "sync");
@@ -351,7 +347,7 @@ int lz_surrogate_gradients(lz_surrogate *s, int n, const uint8_t *planes,
                                hipMemcpyHostToDevice, s->stream), "copy planes");
     if (!rc) rc = s->hip(hipMemcpyAsync(s->y, targets, n * sizeof(float),
                                         hipMemcpyHostToDevice, s->stream), "copy y");
-    if (!rc) rc = forward(s, n, s->planes, s->win, s->stream);
+    if (!rc) rc = forward(s, n, s->planes, s->win, true, s->stream);
     if (!rc) rc = backward(s, n, s->planes, s->y, s->stream);
     if (!rc && grad)
         rc = s->hip(hipMemcpyAsync(grad, s->g, layout().total * sizeof(float),
@@ -372,7 +368,7 @@ int lz_surrogate_train_step_device(lz_surrogate *s, int n,
     std::lock_guard<std::mutex> g(s->mu);
     hipStream_t st = (hipStream_t)stream;  // NULL: the default stream
     rc = join(s, s->stream, st);
-    if (!rc) rc = forward(s, n, planes, nullptr, st);
+    if (!rc) rc = forward(s, n, planes, nullptr, true, st);
     if (!rc) rc = backward(s, n, planes, targets, st);
     if (!rc) {
         s->step++;

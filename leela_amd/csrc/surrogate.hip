@@ -1,19 +1,31 @@
 // surrogate.hip — training and inference kernels of the learned playout
 // surrogate (network in lz_surrogate.h).
 //
-// Convolution (forward and backward-data) — sg_conv
-//   One workgroup per board, 4 waves. The input map is staged into LDS as a
-//   21x21 BF16 HWC tile with a zero halo (pixel stride cin + 8 staggers
-//   pixels across banks). Implicit GEMM D[64 x 368] = A[64 x 9cin] B, K
-//   tap-major, 32 channels per v_mfma_f32_16x16x32_bf16 k-step. A (weights)
-//   is pre-packed in fragment order [k-step][m-tile][lane][8]: one 16-byte
-//   global load per lane (L1/L2 resident). Wave w owns pixel tiles w, w+4,
-//   ... (6 or 5 of the 23) for all 64 output channels. The FP32 epilogue
-//   adds bias and residual, applies ELU (forward) or multiplies by ELU's
-//   derivative taken from the stored forward activation (backward), and
-//   stores BF16 quads.
-//   Backward-data is the same kernel: dX = conv(dY; W') with
-//   W'[c][o][tap] = W[o][c][8 - tap] (taps flipped), packed by pack_conv.
+// Forward — sg_fwd
+//   The whole network for one board per workgroup in one launch: the board
+//   stays in LDS as a zero-haloed BF16 HWC tile (lz_conv_tile.h's layout)
+//   through all 13 convs, each an implicit GEMM on
+//   v_mfma_f32_16x16x32_bf16 with packed weights from L2 (sg_pack), then
+//   the FP32 head. Every conv output also goes to its map in HBM (the
+//   backward pass and read_map take them from there) and nothing is read
+//   back: residuals stay in the registers of the lanes that formed them. The
+//   FP32 epilogue adds bias and residual and applies ELU.
+//   Bound: MFMA and its operand reads from n = 512 up (333 MFLOP a board),
+//   with the maps' stores (0.6 MB a board) beside them; one conv's latency,
+//   13 times, below one board per CU. At n = 4096: 1.32 ms (1.03 PFLOP/s;
+//   1.09 ms with the stores taken out), against 3.37 ms for one launch per
+//   conv with its input staged from HBM each time. Residuals read back from
+//   HBM instead of kept in registers cost 0.7 ms of the 4096, stores of 8
+//   bytes straight from the accumulators 0.4 ms.
+//
+// Backward-data — sg_conv
+//   One workgroup per board, 4 waves. The gradient map is staged into LDS as
+//   a 21x21 BF16 HWC tile with a zero halo (pixel stride 72 staggers pixels
+//   across banks). Wave w owns pixel tiles w, w+4, ... (6 or 5 of the 23)
+//   for all 64 output channels. dX = conv(dY; W') with
+//   W'[c][o][tap] = W[o][c][8 - tap] (taps flipped), packed by sg_pack; the
+//   epilogue adds the skip's gradient, multiplies by ELU's derivative taken
+//   from the stored forward activation, and stores BF16 quads.
 //
 // Weight gradient — sg_wgrad
 //   dW[o][c][tap] = sum over boards and pixels of e[p][o] x[p + tap][c]:
@@ -27,13 +39,13 @@
 //
 // Head (ELU activations), loss, Adam: FP32, small kernels (the head is
 // 0.2% of the FLOPs).
+#include "lz_conv_tile.h"
 #include "lz_surrogate.h"
 
 namespace lz {
 namespace sg {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
@@ -44,6 +56,11 @@ constexpr int KF = 416;                   // 19 x 21 frame, 13 k-steps of 32
 constexpr int KFP = KF + 8;               // LDS row pitch (bank stagger)
 constexpr int kThreads = 256;
 constexpr int kMaxChunks = 64;
+// Batches of at most this many boards (one per CU) use eight waves a board:
+// 95 us up to n = 200 and 102 at 256, against 122-124 with four; from 257 on
+// a CU holds two boards and four waves each are faster (152 against 173 us
+// at 257, 332 against 354 at 1024).
+constexpr int kWideBoards = 256;
 
 __device__ inline f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -66,34 +83,246 @@ __device__ inline float wave_sum(float v) {
 int chunks_for(int n) { return n < kMaxChunks ? n : kMaxChunks; }
 
 // ---- weight packing --------------------------------------------------------
-template <int CIN, bool BWD>
-__global__ __launch_bounds__(kThreads) void sg_pack(const float *__restrict__ w,
-                                                    __bf16 *__restrict__ wpk) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= 9 * CIN * kCh) return;
-    const int e = i & 7, lane = (i >> 3) & 63, mt = (i >> 9) & 3, ks = i >> 11;
-    const int k = ks * 32 + (lane >> 4) * 8 + e;
-    const int row = mt * 16 + (lane & 15);
-    float v;
-    if (!BWD) {
-        const int tap = k / CIN, c = k % CIN;
-        v = w[(row * CIN + c) * 9 + tap];
-    } else {
-        // Row = forward input channel; k = (tap', forward output channel).
-        const int tap = k / kCh, o = k % kCh;
-        v = w[(o * kCh + row) * 9 + (8 - tap)];
+// All convs' MFMA A-operands, forward and (64 -> 64 only) backward-data, in
+// one launch: 25 launches of 9 us of tiny work each were 0.12 ms of a
+// training step. Blocks of the forward weights first, layer by layer, then
+// the backward ones; a thread forms one fragment's 8 values.
+constexpr int kPack0 = 9 * 32 * kCh / 8 / kThreads;   // blocks of layer 0
+constexpr int kPackL = 9 * kCh * kCh / 8 / kThreads;  // of any other
+static_assert(kPack0 * 8 * kThreads == 9 * 32 * kCh &&
+                  kPackL * 8 * kThreads == 9 * kCh * kCh, "whole blocks");
+
+__global__ __launch_bounds__(kThreads) void sg_pack(PackArgs a) {
+    int blk = blockIdx.x, l = 0, cin = 32;
+    bool bwd = false;
+    if (blk >= kPack0) {
+        blk -= kPack0;
+        l = 1 + blk / kPackL;
+        blk %= kPackL;
+        cin = kCh;
+        if (l >= kNConv) {
+            l -= kNConv - 1;
+            bwd = true;
+        }
     }
-    wpk[i] = (__bf16)v;
+    const float *w = a.w[l];
+    const int i = blk * kThreads + threadIdx.x;
+    const int lane = i & 63, mt = (i >> 6) & 3, ks = i >> 8;
+    const int k = ks * 32 + (lane >> 4) * 8;
+    const int row = mt * 16 + (lane & 15);
+    const int tap = k / cin, c = k % cin;  // 8 values: one tap
+    bf16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        // Backward: row = forward input channel, c = forward output channel.
+        v[e] = (__bf16)(bwd ? w[((c + e) * kCh + row) * 9 + (8 - tap)]
+                            : w[(row * cin + c + e) * 9 + tap]);
+    reinterpret_cast<bf16x8 *>(bwd ? a.wb[l] : a.wf[l])[i] = v;
 }
 
-// ---- convolution -------------------------------------------------------------
-template <int CIN, bool BWD>
+// ---- the forward pass ---------------------------------------------------------
+constexpr int kPS = kCh + 16;                    // pixel stride, trunk tile
+constexpr int kInPS = 48;                        // of the 32 input planes
+constexpr int kRP = HS * kPS + row_pad(kPS, 2);  // row pitch
+constexpr int kInRP = HS * kInPS + row_pad(kInPS, 2);
+constexpr int kTile = HS * kRP;
+static_assert(kInRP <= kRP && kTile % 8 == 0, "the input fits the tile");
+
+// The lane's pixel offsets in its wave's column tiles: window origins in the
+// trunk tile (pb) and the pixel index (pix, -1 past the board).
+__device__ __forceinline__ void sg_geom(int wn, int lane, int (&pb)[kNT],
+                                        int (&pix)[kNT]) {
+#pragma unroll
+    for (int t = 0; t < kNT; t++) {
+        const int j = (wn * kNT + t) * 16 + (lane & 15);
+        pix[t] = j < P ? j : -1;
+        // A lane past the board reads the pixel a multiple of 16 before it.
+        const int jj = j < P ? j : j - ((j - P) / 16 + 1) * 16;
+        pb[t] = (jj / S) * kRP + (jj % S) * kPS;
+    }
+}
+
+// Epilogue of a forward conv (bias in the accumulators): + residual, ELU,
+// BF16 into the tile. acc's lane holds four consecutive channels of one
+// pixel per fragment. keep: the lane's outputs of the last even conv, which
+// are the residual of an even conv (kRes) and are replaced by its outputs
+// (kKeep).
+template <bool kRes, bool kKeep, int MTW>
+__device__ __forceinline__ void sg_store_fwd(__bf16 *tile,
+                                             const f32x4 (&acc)[MTW][kNT],
+                                             bf16x4 (&keep)[MTW][kNT],
+                                             int mt0, const int (&pb)[kNT],
+                                             const int (&pix)[kNT], int lane) {
+    const int g4 = (lane >> 4) * 4;
+#pragma unroll
+    for (int m = 0; m < MTW; m++) {
+        const int o = (mt0 + m) * 16 + g4;
+#pragma unroll
+        for (int t = 0; t < kNT; t++) {
+            bf16x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                v[r] = (__bf16)elu_operand(
+                    kRes ? acc[m][t][r] + (float)keep[m][t][r] : acc[m][t][r]);
+            if (kKeep) keep[m][t] = v;
+            if (pix[t] >= 0)
+                *(bf16x4 *)(tile + pb[t] + kRP + kPS + o) = v;
+        }
+    }
+}
+
+// Copies the tile's board to its map in HBM, 16 bytes a lane (T threads).
+// kStream: past the caches, for maps that no kernel of the call reads. Four
+// stores at a time where registers are short (T = 256).
+template <int T, bool kStream>
+__device__ __forceinline__ void sg_copy_out(const __bf16 *tile, __bf16 *map,
+                                            int tid) {
+    constexpr int kUnroll = T > kThreads ? 6 : 4;
+#pragma unroll kUnroll
+    for (int k = 0; k < (P * 8 + T - 1) / T; k++) {
+        const int i = tid + k * T, p = i >> 3;
+        if (i >= P * 8) break;
+        const bf16x8 v = *(const bf16x8 *)(tile + (p / S + 1) * kRP +
+                                           (p % S + 1) * kPS + (i & 7) * 8);
+        if (kStream)
+            __builtin_nontemporal_store(v, (bf16x8 *)(map + i * 8));
+        else
+            *(bf16x8 *)(map + i * 8) = v;
+    }
+}
+
+// kWM waves split the output channels, four the pixels. kWM = 1: two
+// workgroups (75 KB of LDS each) per CU; kWM = 2 halves a board's latency
+// where a CU holds one board only.
+template <int kWM, bool kStream>
+__global__ __launch_bounds__(kWM * kThreads, 2) void sg_fwd(
+    const uint8_t *__restrict__ planes, FwdArgs a, uint16_t *act,
+    size_t map_elems, const float *__restrict__ hp,
+    float *__restrict__ s_out, float *__restrict__ f_out,
+    float *__restrict__ t_out, float *__restrict__ win) {
+    constexpr int T = kWM * kThreads, W = kWM * 4;
+    constexpr int MT = kCh / 16, MTW = MT / kWM;
+    __shared__ __attribute__((aligned(16))) __bf16 tile[kTile];
+    __shared__ float s[P];
+    __shared__ float f[kHid];
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int mt0 = (w / kWN) * MTW;
+    const bf16x8 zero8 = {};
+    __bf16 *maps = (__bf16 *)act + (size_t)b * P * kCh;
+
+    // The planes with a zero halo: a thread takes 8 planes of a point.
+    const uint8_t *pl = planes + (size_t)b * 32 * P;
+    for (int i = tid; i < HP * 4; i += T) {
+        const int hpx = i % HP, c8 = i / HP;
+        const int y = hpx / HS - 1, x = hpx % HS - 1;
+        bf16x8 v = zero8;
+        if (y >= 0 && y < S && x >= 0 && x < S) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[e] = (__bf16)(float)pl[(c8 * 8 + e) * P + y * S + x];
+        }
+        *(bf16x8 *)(tile + (y + 1) * kInRP + (x + 1) * kInPS + c8 * 8) = v;
+    }
+    int pb[kNT], pix[kNT];
+    sg_geom(w % kWN, lane, pb, pix);
+    __syncthreads();
+    bf16x4 keep[MTW][kNT];
+    {
+        f32x4 acc[MTW][kNT];
+        int pbi[kNT];
+#pragma unroll
+        for (int t = 0; t < kNT; t++)
+            pbi[t] = pb[t] / kRP * kInRP + pb[t] % kRP / kPS * kInPS;
+        conv_tile<__bf16, 3, 32, MT, MTW, kInPS>(
+            tile, (const bf16x8 *)a.w[0], acc, pbi, kInRP, mt0, lane, a.b[0]);
+        __syncthreads();
+        for (int i = tid * 8; i < kTile; i += T * 8)
+            *(bf16x8 *)(tile + i) = zero8;
+        __syncthreads();
+        sg_store_fwd<false, true, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        __syncthreads();
+    }
+    // The map of a conv's input goes out between its MFMAs and its epilogue:
+    // loads and stores retire in order, so stores ahead of a conv would
+    // hold up its weight loads, and here the epilogue's math covers them.
+    for (int l = 1; l < kNConv; l += 2) {
+        f32x4 acc[MTW][kNT];
+        conv_tile<__bf16, 3, kCh, MT, MTW, kPS>(
+            tile, (const bf16x8 *)a.w[l], acc, pb, kRP, mt0, lane, a.b[l]);
+        sg_copy_out<T, kStream>(tile, maps + (l - 1) * map_elems, tid);
+        __syncthreads();
+        sg_store_fwd<false, false, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        __syncthreads();
+        conv_tile<__bf16, 3, kCh, MT, MTW, kPS>(
+            tile, (const bf16x8 *)a.w[l + 1], acc, pb, kRP, mt0, lane,
+            a.b[l + 1]);
+        sg_copy_out<T, kStream>(tile, maps + l * map_elems, tid);
+        __syncthreads();
+        sg_store_fwd<true, true, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        __syncthreads();
+    }
+    sg_copy_out<T, kStream>(tile, maps + (kNConv - 1) * map_elems, tid);
+
+    // Head, FP32. hp: wh[64], bh, F1[64][361], c1[64], F2[64], c2.
+    const float *wh = hp, *F1 = hp + kCh + 1;
+    const float *c1 = F1 + kHid * P, *F2 = c1 + kHid;
+    for (int p = tid; p < P; p += T) {
+        const bf16x8 *hv = (const bf16x8 *)(tile + (p / S + 1) * kRP +
+                                            (p % S + 1) * kPS);
+        float d = hp[kCh];
+#pragma unroll
+        for (int c8 = 0; c8 < 8; c8++) {
+            const bf16x8 v = hv[c8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) d += wh[c8 * 8 + k] * (float)v[k];
+        }
+        d = elu(d);
+        s[p] = d;
+        s_out[(size_t)b * P + p] = d;
+    }
+    __syncthreads();
+    // A wave's kHid / W rows of F1 side by side: one wait for the loads of
+    // all of them per 64 points.
+    constexpr int J = kHid / W;
+    float d[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) d[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < (P + 63) / 64; i++) {
+        const int p = i * 64 + lane;
+        if (p < P) {
+            const float sp = s[p];
+#pragma unroll
+            for (int j = 0; j < J; j++) d[j] += F1[(w * J + j) * P + p] * sp;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const float v = wave_sum(d[j]);
+        if (lane == j) {
+            const float fj = elu(v + c1[w * J + j]);
+            f[w * J + j] = fj;
+            f_out[(size_t)b * kHid + w * J + j] = fj;
+        }
+    }
+    __syncthreads();
+    if (w == 0) {
+        const float v = wave_sum(F2[lane] * f[lane]);
+        if (lane == 0) {
+            const float t = tanhf(v + F2[kHid]);
+            t_out[b] = t;
+            if (win) win[b] = 0.5f * (1.f + t);
+        }
+    }
+}
+
+// ---- backward-data convolution ------------------------------------------------
 __global__ __launch_bounds__(kThreads, 2) void sg_conv(
-    const void *__restrict__ in, const bf16x8 *__restrict__ wpk,
-    const float *__restrict__ bias, const __bf16 *__restrict__ res,
-    const __bf16 *__restrict__ mask, __bf16 *__restrict__ out) {
-    constexpr int PS = CIN + 8;
-    constexpr int C8 = CIN / 8;
+    const __bf16 *__restrict__ in, const bf16x8 *__restrict__ wpk,
+    const __bf16 *__restrict__ res, const __bf16 *__restrict__ mask,
+    __bf16 *__restrict__ out) {
+    constexpr int PS = kCh + 8;
+    constexpr int C8 = kCh / 8;
     __shared__ __attribute__((aligned(16))) __bf16 tile[HP * PS];
     const int b = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -105,20 +334,11 @@ __global__ __launch_bounds__(kThreads, 2) void sg_conv(
         if (hy == 0 || hy == HS - 1 || hx == 0 || hx == HS - 1)
             *(bf16x8 *)&tile[hp * PS + c8 * 8] = zero8;
     }
-    if (CIN == 32) {
-        const uint8_t *pl = (const uint8_t *)in + (size_t)b * 32 * P;
-        for (int i = tid; i < 32 * P; i += kThreads) {
-            const int c = i / P, p = i % P;
-            const int y = p / S, x = p % S;
-            tile[((y + 1) * HS + x + 1) * PS + c] = (__bf16)(float)pl[i];
-        }
-    } else {
-        const bf16x8 *src = (const bf16x8 *)in + (size_t)b * P * C8;
-        for (int i = tid; i < P * C8; i += kThreads) {
-            const int p = i / C8, c8 = i % C8;
-            const int y = p / S, x = p % S;
-            *(bf16x8 *)&tile[((y + 1) * HS + x + 1) * PS + c8 * 8] = src[i];
-        }
+    const bf16x8 *src = (const bf16x8 *)in + (size_t)b * P * C8;
+    for (int i = tid; i < P * C8; i += kThreads) {
+        const int p = i / C8, c8 = i % C8;
+        const int y = p / S, x = p % S;
+        *(bf16x8 *)&tile[((y + 1) * HS + x + 1) * PS + c8 * 8] = src[i];
     }
     __syncthreads();
 
@@ -135,9 +355,9 @@ __global__ __launch_bounds__(kThreads, 2) void sg_conv(
         for (int mt = 0; mt < 4; mt++) acc[jj][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int kq = (lane >> 4) * 8;
-    constexpr int KS = 9 * CIN / 32;
+    constexpr int KS = 9 * kCh / 32;
     for (int ks = 0; ks < KS; ks++) {
-        const int tap = (ks * 32) / CIN, c0 = (ks * 32) % CIN;
+        const int tap = (ks * 32) / kCh, c0 = (ks * 32) % kCh;
         const int off = (tap / 3 - 1) * HS + (tap % 3 - 1);
         bf16x8 a[4];
 #pragma unroll
@@ -164,27 +384,16 @@ __global__ __launch_bounds__(kThreads, 2) void sg_conv(
             float v[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = acc[jj][mt][r];
-            if (!BWD) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) v[r] += bias[o + r];
-            }
             if (res) {
                 const bf16x4 rv = *(const bf16x4 *)(res + at);
 #pragma unroll
                 for (int r = 0; r < 4; r++) v[r] += (float)rv[r];
             }
-            if (!BWD) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = elu(v[r]);
-            } else if (mask) {
-                const bf16x4 mv = *(const bf16x4 *)(mask + at);
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    v[r] *= elu_grad((float)mv[r]);
-            }
+            const bf16x4 mv = *(const bf16x4 *)(mask + at);
             bf16x4 ov;
 #pragma unroll
-            for (int r = 0; r < 4; r++) ov[r] = (__bf16)v[r];
+            for (int r = 0; r < 4; r++)
+                ov[r] = (__bf16)(v[r] * elu_grad((float)mv[r]));
             *(bf16x4 *)(out + at) = ov;
         }
     }
@@ -294,54 +503,7 @@ __global__ __launch_bounds__(kThreads) void sg_wgrad_reduce(
     }
 }
 
-// ---- head ------------------------------------------------------------------
-// hp: wh[64], bh, F1[64][361], c1[64], F2[64], c2.
-__global__ __launch_bounds__(kThreads) void sg_head_fwd(
-    const __bf16 *__restrict__ h, const float *__restrict__ hp,
-    float *__restrict__ s_out, float *__restrict__ f_out,
-    float *__restrict__ t_out, float *__restrict__ win) {
-    __shared__ float s[P];
-    __shared__ float f[kHid];
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const float *wh = hp, *F1 = hp + kCh + 1;
-    const float *c1 = F1 + kHid * P, *F2 = c1 + kHid;
-    const float bh = hp[kCh], c2 = F2[kHid];
-    for (int p = tid; p < P; p += kThreads) {
-        const bf16x8 *hv = (const bf16x8 *)(h + ((size_t)b * P + p) * kCh);
-        float d = bh;
-#pragma unroll
-        for (int c8 = 0; c8 < 8; c8++) {
-            const bf16x8 v = hv[c8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) d += wh[c8 * 8 + k] * (float)v[k];
-        }
-        d = elu(d);
-        s[p] = d;
-        s_out[(size_t)b * P + p] = d;
-    }
-    __syncthreads();
-    for (int jj = 0; jj < kHid / 4; jj++) {
-        const int j = w * (kHid / 4) + jj;
-        float d = 0.f;
-        for (int p = lane; p < P; p += 64) d += F1[j * P + p] * s[p];
-        d = wave_sum(d);
-        if (lane == 0) {
-            d = elu(d + c1[j]);
-            f[j] = d;
-            f_out[(size_t)b * kHid + j] = d;
-        }
-    }
-    __syncthreads();
-    if (w == 0) {
-        const float d = wave_sum(F2[lane] * f[lane]);
-        if (lane == 0) {
-            const float t = tanhf(d + c2);
-            t_out[b] = t;
-            if (win) win[b] = 0.5f * (1.f + t);
-        }
-    }
-}
-
+// ---- head, backward ---------------------------------------------------------
 constexpr int kF1 = kHid * P;                     // 23,104
 constexpr int kF1PerThread = (kF1 + kThreads - 1) / kThreads;  // 91
 constexpr int kHeadPart = kHeadParams + 1;        // + loss
@@ -462,36 +624,32 @@ int blocks(long long count) { return (int)((count + kThreads - 1) / kThreads); }
 
 }  // namespace
 
-hipError_t pack_conv(const float *w, uint16_t *wpk, int cin, bool bwd,
-                     hipStream_t stream) {
-    const int g = blocks(9LL * cin * kCh);
-    __bf16 *o = (__bf16 *)wpk;
-    if (cin == 32 && !bwd)
-        sg_pack<32, false><<<g, kThreads, 0, stream>>>(w, o);
-    else if (cin == kCh && !bwd)
-        sg_pack<kCh, false><<<g, kThreads, 0, stream>>>(w, o);
-    else if (cin == kCh && bwd)
-        sg_pack<kCh, true><<<g, kThreads, 0, stream>>>(w, o);
-    else
-        return hipErrorInvalidValue;
+hipError_t pack(const PackArgs &a, hipStream_t stream) {
+    sg_pack<<<kPack0 + 2 * (kNConv - 1) * kPackL, kThreads, 0, stream>>>(a);
     return hipGetLastError();
 }
 
-hipError_t conv(const void *in, int cin, const uint16_t *wpk,
-                const float *bias, const uint16_t *res, const uint16_t *mask,
-                uint16_t *out, int n, bool bwd, hipStream_t stream) {
+hipError_t forward(const uint8_t *planes, const FwdArgs &a, uint16_t *act,
+                   size_t map_elems, const float *hp, float *s, float *f,
+                   float *t, float *win, int n, bool train,
+                   hipStream_t stream) {
     if (n <= 0) return hipSuccess;
-    const bf16x8 *w = (const bf16x8 *)wpk;
-    const __bf16 *r = (const __bf16 *)res, *m = (const __bf16 *)mask;
-    __bf16 *o = (__bf16 *)out;
-    if (cin == 32 && !bwd)
-        sg_conv<32, false><<<n, kThreads, 0, stream>>>(in, w, bias, r, m, o);
-    else if (cin == kCh && !bwd)
-        sg_conv<kCh, false><<<n, kThreads, 0, stream>>>(in, w, bias, r, m, o);
-    else if (cin == kCh && bwd)
-        sg_conv<kCh, true><<<n, kThreads, 0, stream>>>(in, w, bias, r, m, o);
-    else
-        return hipErrorInvalidValue;
+    // One board per CU or fewer: eight waves on each.
+    const int wm = n <= kWideBoards ? 2 : 1;
+    const auto fn = wm == 2 ? (train ? sg_fwd<2, false> : sg_fwd<2, true>)
+                            : (train ? sg_fwd<1, false> : sg_fwd<1, true>);
+    fn<<<n, wm * kThreads, 0, stream>>>(planes, a, act, map_elems, hp, s, f, t,
+                                        win);
+    return hipGetLastError();
+}
+
+hipError_t conv_bwd(const uint16_t *e, const uint16_t *wpk,
+                    const uint16_t *res, const uint16_t *mask, uint16_t *out,
+                    int n, hipStream_t stream) {
+    if (n <= 0) return hipSuccess;
+    sg_conv<<<n, kThreads, 0, stream>>>(
+        (const __bf16 *)e, (const bf16x8 *)wpk, (const __bf16 *)res,
+        (const __bf16 *)mask, (__bf16 *)out);
     return hipGetLastError();
 }
 
@@ -518,14 +676,6 @@ hipError_t wgrad(const void *in, int cin, const uint16_t *e, float *part,
     } else {
         return hipErrorInvalidValue;
     }
-    return hipGetLastError();
-}
-
-hipError_t head_fwd(const uint16_t *h, const float *hp, float *s, float *f,
-                    float *t, float *win, int n, hipStream_t stream) {
-    if (n <= 0) return hipSuccess;
-    sg_head_fwd<<<n, kThreads, 0, stream>>>((const __bf16 *)h, hp, s, f, t,
-                                            win);
     return hipGetLastError();
 }
 

@@ -88,6 +88,31 @@ def test_forward_matches_oracle(sur):
     np.testing.assert_array_equal(sur.predict(planes[5:9]), win[5:9])
 
 
+@pytest.mark.parametrize("n", [1, 3, 256, 257])
+def test_forward_is_the_same_in_every_batch_size(n):
+    """Batches of up to one board per CU run eight waves a board, larger ones
+    four: every output is formed by the same operations in the same order,
+    so a board's maps and win rate are the same bits in any batch; and the
+    first and last board match the oracle (bar as above)."""
+    print(f"surrogate forward: {n} positions, seeds 2500..", flush=True)
+    planes = _value_planes(n, 2500)
+    s = Surrogate(0, max_batch=300, seed=3)
+    try:
+        s.set_params(_random_params(3))
+        flat = s.params().astype(np.float64)
+        more = np.concatenate([planes, _value_planes(300 - n, 9000)])
+        want = s.predict(more)[:n]
+        maps = [s.read_map(0, l, 300)[:n] for l in (0, 1, 12)]
+        np.testing.assert_array_equal(s.predict(planes), want)
+        for l, m in zip((0, 1, 12), maps):
+            np.testing.assert_array_equal(s.read_map(0, l, n), m)
+    finally:
+        s.close()
+    ends = sorted({0, n - 1})
+    t16, _ = orc.forward(flat, planes[ends], bf16_points=True)
+    assert np.abs(want[ends] - (1 + t16) / 2).max() < 1e-2
+
+
 def test_gradients_match_oracle(sur):
     print("surrogate gradients: 6 positions, seeds 700..", flush=True)
     planes = _value_planes(6, 700)
