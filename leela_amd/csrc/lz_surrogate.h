@@ -53,29 +53,39 @@ hipError_t forward(const uint8_t *planes, const FwdArgs &a, uint16_t *act,
                    float *t, float *win, int n, bool train,
                    hipStream_t stream);
 
-// Backward-data of one 64 -> 64 conv over n boards: out = (conv(e) + res)
-// times ELU's derivative at the activation mask. res may be null. Maps BF16
-// [n][361][64].
-hipError_t conv_bwd(const uint16_t *e, const uint16_t *wpk,
-                    const uint16_t *res, const uint16_t *mask, uint16_t *out,
-                    int n, hipStream_t stream);
-
-// Weight and bias gradient of one conv: gW (OIHW) and gb are written (not
-// accumulated). e: BF16 [n][361][64] gradient at the conv's pre-activation;
-// in: the conv's input (u8 planes when cin == 32). part must hold
-// wgrad_part_floats(cin, n) floats.
-size_t wgrad_part_floats(int cin, int n);
-hipError_t wgrad(const void *in, int cin, const uint16_t *e, float *part,
-                 float *gW, float *gb, int n, hipStream_t stream);
-
-// Loss mean_n (t - (2y - 1))^2, head gradients (into ghp, written), the
-// BF16 gradient e [n][361][64] at the last conv's pre-activation, and the
-// loss into *loss (device). part must hold head_part_floats(n) floats.
-size_t head_part_floats(int n);
-hipError_t head_bwd(const uint16_t *h, const float *hp, const float *s,
-                    const float *f, const float *t, const float *y,
-                    uint16_t *e, float *part, float *ghp, float *loss, int n,
+// The backward pass to every pre-activation, for boards b0 .. b0 + n - 1 of
+// a batch of `total` (loss mean_n (t - (2y - 1))^2) after forward(): the
+// gradient at conv l's pre-activation into e + l * e_elems (BF16
+// [n][361][64], board b0 first), and each board's kHeadRow floats of head
+// gradients into hpart (indexed by board, as act, s, f, t and y are). w:
+// packed backward-data weights (from conv 1 on).
+constexpr int kHeadRow = 196;
+struct BwdArgs {
+    const uint16_t *w[kNConv];
+};
+hipError_t backward(const BwdArgs &a, const uint16_t *act, size_t map_elems,
+                    const float *hp, const float *s, const float *f,
+                    const float *t, const float *y, uint16_t *e,
+                    size_t e_elems, float *hpart, int b0, int n, int total,
                     hipStream_t stream);
+
+// Weight and bias gradients of every conv from n boards: e[l] its gradient
+// maps, in[l] its input (u8 planes for conv 0). Written to w[l] (OIHW) and
+// b[l], or added when `add`. With total > 0 (the last boards of a batch of
+// `total`) also the head's gradients into ghp and the mean loss into *loss
+// (device), from hpart and s. part must hold part_floats(n) floats.
+struct WgradArgs {
+    const void *in[kNConv];
+    const uint16_t *e[kNConv];
+    const void *zeros;  // 16 zero bytes
+};
+struct GradArgs {
+    float *w[kNConv], *b[kNConv];
+};
+size_t part_floats(int n);
+hipError_t wgrad(const WgradArgs &a, float *part, int n, const GradArgs &ga,
+                 bool add, const float *hpart, const float *s, int total,
+                 float *ghp, float *loss, hipStream_t stream);
 
 // Adam (Kingma & Ba 2015, Algorithm 1) over count parameters; c1 = 1 -
 // beta1^step, c2 = 1 - beta2^step.

@@ -6,9 +6,10 @@
 //   params / grads / Adam m / Adam v   4 x 484,930 FP32
 //   packed weights                     13 forward + 12 backward-data convs
 //   activations                        13 x B x 361 x 64 BF16 (all kept)
-//   conv-gradient maps                 3 x B x 361 x 64 BF16 (rotating)
+//   conv-gradient maps                 13 x min(B, 1024) x 361 x 64 BF16
 //   head saves s/f/t                   B x (361 + 64 + 1) FP32
-//   partial sums                       max of the wgrad and head partials
+//   partial sums                       weight gradients of up to 39 chunks of
+//                                      boards, head gradients per board
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -27,6 +28,10 @@ using namespace lz::sg;
 
 constexpr uint32_t kMagic = 0x47535a4c;  // "LZSG"
 constexpr uint32_t kVersion = 1;
+// The backward pass takes at most this many boards at a time (two rounds of
+// two boards per CU), so that its 13 gradient maps do not grow with the
+// batch: 0.6 GB at the most.
+constexpr int kBwdBoards = 1024;
 
 struct Layout {
     size_t w[kNConv], b[kNConv], head, total;
@@ -58,11 +63,12 @@ struct lz_surrogate {
     std::string err;
     float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     uint16_t *wf[kNConv] = {}, *wb[kNConv] = {};
-    uint16_t *act = nullptr, *e[3] = {};
+    uint16_t *act = nullptr, *e = nullptr;
     uint16_t *ekeep = nullptr;   // all 13 gradient maps (inspection mode)
     float *s = nullptr, *f = nullptr, *t = nullptr, *y = nullptr;
-    float *loss = nullptr, *part = nullptr;
+    float *loss = nullptr, *part = nullptr, *hpart = nullptr;
     uint8_t *planes = nullptr;   // staging of the host entry points
+    uint8_t *zeros = nullptr;    // the weight gradients' zero block
     float *win = nullptr;
     hipEvent_t ev = nullptr;
     long long step = 0;
@@ -79,10 +85,8 @@ struct lz_surrogate {
     }
     size_t map_elems() const { return (size_t)max_batch * kP * kCh; }
     uint16_t *act_of(int l) const { return act + (size_t)l * map_elems(); }
-    // Gradient map at the pre-activation of conv l. Three rotating maps
-    // suffice: computing map l-1 reads maps l and l+1.
-    uint16_t *emap(int l) const {
-        return ekeep ? ekeep + (size_t)l * map_elems() : e[l % 3];
+    int bwd_boards() const {
+        return max_batch < kBwdBoards ? max_batch : kBwdBoards;
     }
 };
 
@@ -96,9 +100,9 @@ hipError_t dalloc(T **ptr, size_t count) {
 void release(lz_surrogate *s) {
     (void)hipSetDevice(s->device);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
-    void *bufs[] = {s->p, s->g, s->m, s->v, s->act, s->e[0], s->e[1], s->e[2],
-                    s->ekeep, s->s, s->f, s->t, s->y, s->loss, s->part,
-                    s->planes, s->win};
+    void *bufs[] = {s->p, s->g, s->m, s->v, s->act, s->e, s->ekeep, s->s, s->f,
+                    s->t, s->y, s->loss, s->part, s->hpart, s->planes, s->win,
+                    s->zeros};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     for (int l = 0; l < kNConv; l++) {
@@ -142,28 +146,43 @@ int forward(lz_surrogate *s, int n, const uint8_t *planes, float *win,
 }
 
 // Backward of the last forward into s->g (written, not accumulated); the
-// mean loss lands in s->loss (device). Map l is the gradient at the
-// pre-activation of conv l: the second conv of a block (even l >= 2) passes
-// map l to its first conv, and the first conv (odd l) adds map l + 1 (the
-// skip) before masking by the block input.
+// mean loss lands in s->loss (device). Parts of kBwdBoards boards, each the
+// gradient maps and then their weight gradients (in inspection mode the maps
+// of all boards are kept).
 int backward(lz_surrogate *s, int n, const uint8_t *planes, const float *y,
              hipStream_t st) {
     const Layout &L = layout();
-    const int last = kNConv - 1;
-    int rc = s->hip(head_bwd(s->act_of(last), s->p + L.head, s->s, s->f, s->t,
-                             y, s->emap(last), s->part, s->g + L.head, s->loss,
-                             n, st), "head_bwd");
-    for (int l = last; !rc && l >= 1; l--) {
-        rc = s->hip(wgrad(s->act_of(l - 1), kCh, s->emap(l), s->part,
-                          s->g + L.w[l], s->g + L.b[l], n, st), "wgrad");
-        if (rc) return rc;
-        const uint16_t *res = (l % 2 == 1) ? s->emap(l + 1) : nullptr;
-        rc = s->hip(conv_bwd(s->emap(l), s->wb[l], res, s->act_of(l - 1),
-                             s->emap(l - 1), n, st), "conv_bwd");
+    BwdArgs ba = {};
+    GradArgs ga = {};
+    for (int l = 0; l < kNConv; l++) {
+        ba.w[l] = s->wb[l];
+        ga.w[l] = s->g + L.w[l];
+        ga.b[l] = s->g + L.b[l];
     }
-    if (rc) return rc;
-    return s->hip(wgrad(planes, 32, s->emap(0), s->part, s->g + L.w[0],
-                        s->g + L.b[0], n, st), "wgrad");
+    const size_t board = (size_t)kP * kCh;
+    for (int b0 = 0; b0 < n; b0 += kBwdBoards) {
+        const int k = n - b0 < kBwdBoards ? n - b0 : kBwdBoards;
+        uint16_t *e = s->ekeep ? s->ekeep + b0 * board : s->e;
+        const size_t e_elems =
+            s->ekeep ? s->map_elems() : (size_t)s->bwd_boards() * board;
+        int rc = s->hip(lz::sg::backward(ba, s->act, s->map_elems(),
+                                         s->p + L.head, s->s, s->f, s->t, y, e,
+                                         e_elems, s->hpart, b0, k, n, st),
+                        "backward");
+        if (rc) return rc;
+        WgradArgs wa = {};
+        wa.zeros = s->zeros;
+        for (int l = 0; l < kNConv; l++) {
+            wa.in[l] = l == 0 ? (const void *)(planes + (size_t)b0 * 32 * kP)
+                              : (const void *)(s->act_of(l - 1) + b0 * board);
+            wa.e[l] = e + l * e_elems;
+        }
+        const bool last = b0 + k == n;
+        rc = s->hip(wgrad(wa, s->part, k, ga, b0 > 0, s->hpart, s->s,
+                          last ? n : 0, s->g + L.head, s->loss, st), "wgrad");
+        if (rc) return rc;
+    }
+    return LZ_OK;
 }
 
 // Orders `to` after the work queued so far on `from`.
@@ -204,11 +223,6 @@ int lz_surrogate_create(lz_surrogate **out, int device, int max_batch,
     s->max_batch = max_batch;
     const Layout &L = layout();
     const size_t B = (size_t)max_batch;
-    size_t part = head_part_floats(max_batch);
-    for (int cin : {32, kCh}) {
-        const size_t w = wgrad_part_floats(cin, max_batch);
-        if (w > part) part = w;
-    }
     bool ok = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) == hipSuccess &&
               hipEventCreateWithFlags(&s->ev, hipEventDisableTiming) == hipSuccess;
     ok = ok && dalloc(&s->p, L.total) == hipSuccess &&
@@ -220,9 +234,12 @@ int lz_surrogate_create(lz_surrogate **out, int device, int max_batch,
          dalloc(&s->f, B * kHid) == hipSuccess &&
          dalloc(&s->t, B) == hipSuccess && dalloc(&s->y, B) == hipSuccess &&
          dalloc(&s->win, B) == hipSuccess && dalloc(&s->loss, 1) == hipSuccess &&
-         dalloc(&s->part, part) == hipSuccess &&
+         dalloc(&s->part, part_floats(s->bwd_boards())) == hipSuccess &&
+         dalloc(&s->hpart, B * kHeadRow) == hipSuccess &&
+         dalloc(&s->zeros, 64) == hipSuccess &&
+         dalloc(&s->e, kNConv * (size_t)s->bwd_boards() * kP * kCh) ==
+             hipSuccess &&
          dalloc(&s->planes, B * 32 * kP) == hipSuccess;
-    for (int i = 0; ok && i < 3; i++) ok = dalloc(&s->e[i], s->map_elems()) == hipSuccess;
     for (int l = 0; ok && l < kNConv; l++) {
         ok = dalloc(&s->wf[l], (size_t)conv_weights(l)) == hipSuccess;
         if (ok && l > 0) ok = dalloc(&s->wb[l], (size_t)conv_weights(l)) == hipSuccess;
@@ -250,7 +267,8 @@ int lz_surrogate_create(lz_surrogate **out, int device, int max_batch,
     ok = hipMemcpy(s->p, h.data(), L.total * sizeof(float),
                    hipMemcpyHostToDevice) == hipSuccess &&
          hipMemset(s->m, 0, L.total * sizeof(float)) == hipSuccess &&
-         hipMemset(s->v, 0, L.total * sizeof(float)) == hipSuccess;
+         hipMemset(s->v, 0, L.total * sizeof(float)) == hipSuccess &&
+         hipMemset(s->zeros, 0, 64) == hipSuccess;
     if (!ok) {
         release(s);
         delete s;
@@ -414,7 +432,8 @@ int lz_surrogate_read_map(lz_surrogate *s, int kind, int layer, int n,
     if (kind == 1 && !s->ekeep)
         return s->fail(LZ_ERR_STATE, "gradient maps are not kept");
     std::lock_guard<std::mutex> g(s->mu);
-    const uint16_t *src = kind == 0 ? s->act_of(layer) : s->emap(layer);
+    const uint16_t *src = kind == 0 ? s->act_of(layer)
+                                    : s->ekeep + (size_t)layer * s->map_elems();
     rc = s->hip(hipStreamSynchronize(s->stream), "sync");
     if (!rc)
         rc = s->hip(hipMemcpy(out, src, (size_t)n * kP * kCh * sizeof(uint16_t),

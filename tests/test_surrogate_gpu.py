@@ -142,6 +142,39 @@ def test_gradients_match_oracle(sur):
     np.testing.assert_array_equal(g, g2)
 
 
+@pytest.mark.parametrize("k", [1, 10, 19, 25, 129, 1025])
+def test_gradient_of_a_batch_is_the_mean_of_its_halves(k):
+    """2k boards against their two halves: the factor 1 / n halves exactly, so
+    every gradient map is the half's to the bit, and the weight gradients
+    differ by the order of FP32 sums only (runs of boards per workgroup, the
+    tail of the last run, and the split of the backward pass at 1024
+    boards). Sums of N = 361 n products by magnitude up to 2k boards:
+    N^(1/2) ulps at random, 2^-24 * sqrt(361 * 2050) = 5e-5 of the largest
+    sum, taken as 1e-4 of the tensor's maximum."""
+    print(f"surrogate gradient: 2 x {k} positions", flush=True)
+    planes = _value_planes(2 * k, 40000 + k)
+    y = np.random.default_rng(k).uniform(0.1, 0.9, 2 * k).astype(np.float32)
+    s = Surrogate(0, max_batch=2 * k, seed=3)
+    try:
+        s.set_params(_random_params(7))
+        loss, g = s.gradients(planes, y)
+        la, ga = s.gradients(planes[:k], y[:k])
+        lb, gb = s.gradients(planes[k:], y[k:])
+        s.keep_maps(True)
+        _, g2 = s.gradients(planes, y)
+    finally:
+        s.close()
+    np.testing.assert_array_equal(g, g2)
+    assert abs(loss - (la + lb) / 2) <= 1e-5 * abs(loss)
+    want = (ga.astype(np.float64) + gb) / 2
+    for name, shape, off in orc.layout():
+        n = int(np.prod(shape))
+        a, b = g[off:off + n], want[off:off + n]
+        assert np.abs(b).max() > 0, name
+        np.testing.assert_allclose(a, b, rtol=0, atol=1e-4 * np.abs(b).max(),
+                                   err_msg=name)
+
+
 def _bf(u16):
     """BF16 bit patterns -> float64."""
     return (u16.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
