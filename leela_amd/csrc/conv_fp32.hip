@@ -1,29 +1,38 @@
 // conv_fp32.hip — the FP32 "plain" form of Leela's policy and value nets.
 //
-// One workgroup computes one board x 64 output channels of a same-padded
-// conv as an implicit GEMM on FP32 MFMA (v_mfma_f32_16x16x4_f32):
-//   D[cout x pixels] = W[cout x cin*k*k] * im2col(X)[cin*k*k x pixels]
-// which is the product the reference forms explicitly with im2col + sgemm
-// (Network.cpp:344-393, Im2Col.h:9-50). The input board is staged in LDS
-// one channel chunk at a time with a zero halo, so the im2col matrix is
-// never materialised: a B-operand element is one LDS read at
-// chunk_offset(c, ky, kx) + pixel_offset(y, x). Channels past cin in the
-// last chunk stage as zeros (their packed weight rows are zero too), so any
-// input channel count works. Bias, the activation (ELU, Network.cpp:
-// 382-392; or ReLU / none for Caffe nets) and an optional batch
+// FP32 convolution on the 16-bit matrix cores (conv_split). Every FP32 value
+// is written as the sum of three BF16 values (round to nearest each time:
+// 8 + 8 + 8 bits and their signs hold the 24 bits exactly, down to 2^-126
+// for the smallest part), and a product is the sum of the six partial
+// products above 2^-25 of it, each exact in FP32:
+//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1 + O(2^-25 a b).
+// Sums are FP32 throughout (v_mfma_f32_16x16x32_bf16 adds 32 products with
+// fewer roundings than an FP32 chain has), activations stay FP32 in memory.
+// Against 64 bits the nets' outputs are no further off than with FP32 MFMA
+// (policy probabilities of 96 boards 3.7e-6 against 5.1e-6, a trained net's
+// logits 3.7e-6 against 4.2e-6). The FP32 matrix unit runs at 1/16 of the
+// BF16 rate, so six products are 2.7 times its peak: 1024 boards through
+// the policy net take 5.06 ms (243 TFLOP/s of FP32 products), against 15.9
+// on FP32 MFMA (77 TFLOP/s of 157).
+//
+// The product is the one that the reference forms with im2col + sgemm
+// (Network.cpp:344-393, Im2Col.h:9-50). Bias, the activation (ELU,
+// Network.cpp:382-392; or ReLU / none for Caffe nets) and an optional batch
 // normalisation of the activated output (Network.cpp:427-448) are fused
-// into the epilogue.
+// into the epilogue. Activations between convs: [n][361][C], C rounded up to
+// 32 channels (the extra ones zero).
+#include <type_traits>
+
+#include "lz_conv_tile.h"
 #include "lz_internal.h"
 
 namespace lz {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kThreads = 256;           // 4 waves
-constexpr int kNTiles = 24;             // 16-pixel tiles: 384 >= 361
-constexpr int kTilesPerWave = kNTiles / 4;
-constexpr int kMTiles = kF32MBlock / 16;
+constexpr int kS = 19, kP = kS * kS;    // the nets' board
 
 __device__ __forceinline__ float elu(float v) {
     return v > 0.0f ? v : (expf(v) - 1.0f);
@@ -35,162 +44,286 @@ __device__ __forceinline__ float activate(float v, int act) {
     return v;
 }
 
-template <int F>
-struct ConvF32Cfg {
-    static constexpr int CK = (F == 5) ? 8 : 16;  // input channels per chunk
-    static constexpr int KC = CK * F * F;         // K rows per chunk
-    static constexpr int SP = kMaxSide + 2 * (F / 2);
-};
+// The three BF16 parts of eight FP32 values. (Values past BF16's largest,
+// 3.39e38, take that as their first part; infinities end up NaN.)
+__device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
+    constexpr float kMax = 3.3895313892515355e38f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const __bf16 h = (__bf16)__builtin_amdgcn_fmed3f(x[e], -kMax, kMax);
+        const float r = x[e] - (float)h;
+        const __bf16 m = (__bf16)r;
+        p[0][e] = h;
+        p[1][e] = m;
+        p[2][e] = (__bf16)(r - (float)m);
+    }
+}
 
-template <int F, typename InT>
-__global__ __launch_bounds__(kThreads) void conv_f32_kernel(
-    const InT *__restrict__ in, const float *__restrict__ wpk,
+// One conv. A workgroup computes a band of R image rows of one board (10
+// rows, NTW = 6, or 5, NTW = 3) for 2 * MTW m-tiles of 16 output channels:
+// its four waves are 2 (channels) x 2 (pixels), each MTW m-tiles x NTW
+// column tiles of 16 pixels. Per chunk of 32 input channels the band's rows
+// and halo are split and staged in LDS, HWC, the parts of a pixel side by
+// side (NB = 3 parts of 32 channels; byte planes are exact in one, NB = 1),
+// then F * F k-steps follow. Weights: [chunk][tap][part][m-tile][lane][8].
+//
+// Bound: the matrix cores, six products a term. The order of the products
+// gives every operand's reload a group of MFMAs or more before its next
+// use. Small pieces (few MFMAs a step) keep F steps of weights on the way
+// and load the next chunk's values under this one's MFMAs (policy net, one
+// board: 310 us without, 216 with).
+template <int F, int NB, int MTW, int NTW>
+__global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
+    const void *__restrict__ in, const bf16x8 *__restrict__ wpk,
     const float *__restrict__ bias, float *__restrict__ out, int cin,
-    int cout, int S, ConvEpilogue epi) {
-    using C = ConvF32Cfg<F>;
-    constexpr int PAD = F / 2;
-    __shared__ float s_in[C::CK * C::SP * C::SP];
-    __shared__ f32x4 s_w4[C::KC * kF32MBlock / 4];
-    __shared__ int s_koff[C::KC];
-    const float *s_w = reinterpret_cast<const float *>(s_w4);
+    int chunks, int cout, int cstride, int mtiles, ConvEpilogue epi) {
+    constexpr int R = NTW == 6 ? 10 : 5, BANDS = (kS + R - 1) / R;
+    constexpr int W = kS + F - 1, PS = NB * 32 + 16;
+    constexpr int RP = W * PS + row_pad(PS, F - 1);
+    constexpr int FF = F * F;
+    constexpr bool kSmall = NTW == 3 && MTW <= 2;
+    // k-steps of weights held (a divisor of F * F, as registers allow).
+    constexpr int D = kSmall && (F == 3 || MTW == 1) ? F : 1;
+    constexpr int TASKS = ((R + F - 1) * W * 4 + kThreads - 1) / kThreads;
+    static_assert(R * kS <= 2 * NTW * 16, "column tiles cover the band");
+    __shared__ __attribute__((aligned(16))) __bf16 tile[(R + F - 1) * RP];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int board = blockIdx.x / BANDS, y0 = blockIdx.x % BANDS * R;
+    const int rows = y0 + R < kS ? R : kS - y0, npx = rows * kS;
+    const int mt0 = (blockIdx.y * 2 + (w & 1)) * MTW;
+    const int g8 = (lane >> 4) * 8;
 
-    const int board = blockIdx.x;
-    const int mb = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int P = S * S;
-    const int SPs = S + 2 * PAD;  // padded side of this board
-    const int plane = SPs * SPs;
-
-    // Offsets of the (c, ky, kx) rows of one chunk inside s_in.
-    for (int i = tid; i < C::KC; i += kThreads) {
-        const int c = i / (F * F), r = i % (F * F);
-        s_koff[i] = c * plane + (r / F) * SPs + (r % F);
+    int pb[NTW], pix[NTW];
+#pragma unroll
+    for (int t = 0; t < NTW; t++) {
+        const int j = ((w >> 1) * NTW + t) * 16 + (lane & 15);
+        pix[t] = j < npx ? y0 * kS + j : -1;
+        // A lane past the band reads a pixel a multiple of 16 before it.
+        const int jj = j < npx ? j : j - ((j - npx) / 16 + 1) * 16;
+        pb[t] = (jj / kS) * RP + (jj % kS) * PS + g8;
     }
-    // Offset of this lane's pixel in each of its wave's N tiles. Columns
-    // past the board read in-bounds garbage and are never stored.
-    int poff[kTilesPerWave];
+    f32x4 acc[MTW][NTW];
 #pragma unroll
-    for (int t = 0; t < kTilesPerWave; t++) {
-        const int j = (wave * kTilesPerWave + t) * 16 + (lane & 15);
-        poff[t] = j < P ? (j / S) * SPs + (j % S) : 0;
-    }
-
-    f32x4 acc[kMTiles][kTilesPerWave];
+    for (int m = 0; m < MTW; m++)
 #pragma unroll
-    for (int m = 0; m < kMTiles; m++)
+        for (int t = 0; t < NTW; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // Weights of k-step s (over chunks and taps), part p, into set d. Tiles
+    // past the last m-tile re-read it and are not stored.
+    const int steps = chunks * FF;
+    int mt[MTW];
 #pragma unroll
-        for (int t = 0; t < kTilesPerWave; t++) acc[m][t] = f32x4{0, 0, 0, 0};
-
-    const InT *src = in + (size_t)board * cin * P;
-    const int K = f32_packed_k(F, cin);  // cin rounded up to whole chunks
-    const f32x4 *wsrc4 = reinterpret_cast<const f32x4 *>(
-        wpk + (size_t)mb * K * kF32MBlock);
-    const int kq = lane >> 4;
-    const int ml = lane & 15;
-
-    for (int c0 = 0; c0 < cin; c0 += C::CK) {
-        __syncthreads();
-        for (int i = tid; i < C::CK * plane; i += kThreads) {
-            const int c = i / plane, r = i % plane;
-            const int y = r / SPs - PAD, x = r % SPs - PAD;
-            float v = 0.0f;
-            if (y >= 0 && y < S && x >= 0 && x < S && c0 + c < cin)
-                v = (float)src[(size_t)(c0 + c) * P + y * S + x];
-            s_in[i] = v;
+    for (int m = 0; m < MTW; m++)
+        mt[m] = (mt0 + m < mtiles ? mt0 + m : mtiles - 1) * 64 + lane;
+    bf16x8 a[D][3][MTW], b[NB][NTW];
+    auto load_a = [&](int d, int s, int p) {
+        s = s < steps ? s : steps - 1;
+        const bf16x8 *at = wpk + (size_t)(s * 3 + p) * mtiles * 64;
+#pragma unroll
+        for (int m = 0; m < MTW; m++) a[d][p][m] = at[mt[m]];
+    };
+    auto load_b = [&](int tap, int p) {
+        tap = tap < FF ? tap : FF - 1;
+        const __bf16 *at = tile + (tap / F) * RP + (tap % F) * PS + p * 32;
+#pragma unroll
+        for (int t = 0; t < NTW; t++)
+            b[p][t] = *(const bf16x8 *)(at + pb[t]);
+    };
+    auto mul = [&](int d, int pa, int pbk) {
+#pragma unroll
+        for (int m = 0; m < MTW; m++)
+#pragma unroll
+            for (int t = 0; t < NTW; t++)
+                acc[m][t] =
+                    Op<__bf16>::mfma(a[d][pa][m], b[pbk][t], acc[m][t]);
+    };
+    // Task k of a chunk's staging: eight channels of a point of the band's
+    // frame (zeros off the board), as values (float input) or one part.
+    auto fetch = [&](int chunk, int k, float (&v)[8]) {
+        const int i = tid + k * kThreads;
+        const int c8 = (i & 3) * 8, q = i >> 2;
+        const int y = y0 - F / 2 + q / W, x = q % W - F / 2;
+        const bool on = q < (R + F - 1) * W && y >= 0 && y < kS && x >= 0 &&
+                        x < kS;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = 0.f;
+        if (!on) return;
+        if (NB == 1) {
+            const int c = chunk * 32 + c8;
+            const uint8_t *src =
+                (const uint8_t *)in + ((size_t)board * cin + c) * kP + y * kS + x;
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (c + e < cin) v[e] = (float)src[e * kP];
+        } else {
+            const f32x4 *src =
+                (const f32x4 *)((const float *)in +
+                                ((size_t)board * kP + y * kS + x) *
+                                    (chunks * 32) +
+                                chunk * 32 + c8);
+            const f32x4 lo = src[0], hi = src[1];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = lo[e];
+                v[4 + e] = hi[e];
+            }
         }
-        const f32x4 *wchunk = wsrc4 + (size_t)c0 * F * F * kF32MBlock / 4;
-        for (int i = tid; i < C::KC * kF32MBlock / 4; i += kThreads)
-            s_w4[i] = wchunk[i];
-        __syncthreads();
+    };
+    auto put = [&](int k, const float (&v)[8]) {
+        const int i = tid + k * kThreads, q = i >> 2;
+        if (q >= (R + F - 1) * W) return;
+        __bf16 *dst = tile + (q / W) * RP + (q % W) * PS + (i & 3) * 8;
+        bf16x8 parts[3];
+        split3(v, parts);
+#pragma unroll
+        for (int p = 0; p < NB; p++) *(bf16x8 *)(dst + p * 32) = parts[p];
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++)
+#pragma unroll
+        for (int p = 0; p < 3; p++) load_a(d, d, p);
 
-        for (int ks = 0; ks < C::KC; ks += 4) {
-            const int k = ks + kq;
-            const int ko = s_koff[k];
-            float a[kMTiles], b[kTilesPerWave];
+    float next[kSmall ? TASKS : 1][8];
+    if constexpr (kSmall) {
 #pragma unroll
-            for (int m = 0; m < kMTiles; m++)
-                a[m] = s_w[k * kF32MBlock + m * 16 + ml];
+        for (int k = 0; k < TASKS; k++) fetch(0, k, next[k]);
+    }
+    for (int chunk = 0; chunk < chunks; chunk++) {
+        __syncthreads();
+        if constexpr (kSmall) {
 #pragma unroll
-            for (int t = 0; t < kTilesPerWave; t++) b[t] = s_in[ko + poff[t]];
+            for (int k = 0; k < TASKS; k++) put(k, next[k]);
+            if (chunk + 1 < chunks) {
 #pragma unroll
-            for (int m = 0; m < kMTiles; m++)
+                for (int k = 0; k < TASKS; k++) fetch(chunk + 1, k, next[k]);
+            }
+        } else {
+            for (int k = 0; k < TASKS; k++) {
+                fetch(chunk, k, next[0]);
+                put(k, next[0]);
+            }
+        }
+        __syncthreads();
 #pragma unroll
-                for (int t = 0; t < kTilesPerWave; t++)
-                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        a[m], b[t], acc[m][t], 0, 0, 0);
+        for (int p = 0; p < NB; p++) load_b(0, p);
+        for (int tap0 = 0; tap0 < FF; tap0 += D) {
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                const int tap = tap0 + d, s = chunk * FF + tap + D;
+                if constexpr (NB == 3) {
+                    mul(d, 0, 2);
+                    load_b(tap + 1, 2);
+                    mul(d, 0, 1);
+                    mul(d, 0, 0);
+                    load_a(d, s, 0);
+                    mul(d, 1, 0);
+                    mul(d, 1, 1);
+                    load_a(d, s, 1);
+                    load_b(tap + 1, 1);
+                    mul(d, 2, 0);
+                    load_a(d, s, 2);
+                    load_b(tap + 1, 0);
+                } else {
+                    mul(d, 0, 0);
+                    load_a(d, s, 0);
+                    mul(d, 1, 0);
+                    load_a(d, s, 1);
+                    mul(d, 2, 0);
+                    load_a(d, s, 2);
+                    load_b(tap + 1, 0);
+                }
+            }
         }
     }
 
-    // D layout of 16x16x4: lane holds rows 4*(lane/16)+r of column lane%16.
-    float *dst = out + (size_t)board * cout * P;
+    // D layout of 16x16 MFMA: lane holds rows 4*(lane/16)+r of column
+    // lane%16: four channels of a pixel.
 #pragma unroll
-    for (int m = 0; m < kMTiles; m++) {
+    for (int m = 0; m < MTW; m++) {
+        const int o = (mt0 + m) * 16 + (lane >> 4) * 4;
+        if (o >= cstride) continue;
+        float bo[4], bm[4], ba[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int o = mb * kF32MBlock + m * 16 + 4 * (lane >> 4) + r;
-            if (o >= cout) continue;
-            const float bo = bias[o];
-            const float bm = epi.bn_mean ? epi.bn_mean[o] : 0.0f;
-            const float ba = epi.bn_mean ? epi.bn_inv_std[o] : 1.0f;
+            const bool on = o + r < cout;
+            bo[r] = on ? bias[o + r] : 0.f;
+            bm[r] = on && epi.bn_mean ? epi.bn_mean[o + r] : 0.f;
+            ba[r] = on && epi.bn_mean ? epi.bn_inv_std[o + r] : 1.f;
+        }
 #pragma unroll
-            for (int t = 0; t < kTilesPerWave; t++) {
-                const int j = (wave * kTilesPerWave + t) * 16 + (lane & 15);
-                if (j >= P) continue;
-                float v = activate(acc[m][t][r] + bo, epi.act);
+        for (int t = 0; t < NTW; t++) {
+            if (pix[t] < 0) continue;
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                v[r] = activate(acc[m][t][r] + bo[r], epi.act);
                 // Network.cpp:445: scale_stddiv * (in - mean).
-                if (epi.bn_mean) v = ba * (v - bm);
-                dst[(size_t)o * P + j] = v;
+                if (epi.bn_mean) v[r] = ba[r] * (v[r] - bm[r]);
+                if (o + r >= cout) v[r] = 0.f;
             }
+            *(f32x4 *)(out + ((size_t)board * kP + pix[t]) * cstride + o) = v;
         }
     }
 }
 
 // ---- 1-channel head convs -------------------------------------------------
+// The 3x3 conv to one channel as a product with the nine taps as rows:
+// d[tap][p] = sum_c w[tap][c] x[p][c] (split as above, 16 rows of which nine
+// are used), then out[p] = sum_tap d[tap][p shifted by the tap]. Every input
+// value is read once, straight into an operand. Weights: [chunk][part]
+// [lane][8], lane = tap + 16 * channel group.
+constexpr int kHeadThreads = 512;
+constexpr int kHeadPix = 368;  // 23 column tiles
 
-constexpr int kHeadCK = 16;
-constexpr int kHeadSP = kMaxSide + 2;
-
-// Computes the activated 3x3 (cin -> 1) conv of one board into
-// s_out[0..P). Each thread owns pixels tid and tid + 256.
-__device__ void head_conv3(const float *__restrict__ src,
-                           const float *__restrict__ w, float b, int cin,
-                           int S, int act, float *s_in, float *s_w,
-                           float *s_out) {
-    const int tid = threadIdx.x;
-    const int P = S * S, SPs = S + 2, plane = SPs * SPs;
-    float acc0 = 0.0f, acc1 = 0.0f;
-    const int p0 = tid, p1 = tid + kThreads;
-    const int o0 = p0 < P ? (p0 / S) * SPs + p0 % S : 0;
-    const int o1 = p1 < P ? (p1 / S) * SPs + p1 % S : 0;
-    for (int c0 = 0; c0 < cin; c0 += kHeadCK) {
-        __syncthreads();
-        for (int i = tid; i < kHeadCK * plane; i += kThreads) {
-            const int c = i / plane, r = i % plane;
-            const int y = r / SPs - 1, x = r % SPs - 1;
-            float v = 0.0f;
-            if (y >= 0 && y < S && x >= 0 && x < S && c0 + c < cin)
-                v = src[(size_t)(c0 + c) * P + y * S + x];
-            s_in[i] = v;
-        }
-        for (int i = tid; i < kHeadCK * 9; i += kThreads)
-            s_w[i] = c0 + i / 9 < cin ? w[c0 * 9 + i] : 0.0f;
-        __syncthreads();
-        for (int c = 0; c < kHeadCK; c++) {
-            const float *pl = s_in + c * plane;
+// The activated conv of one board into s_out[0..361).
+__device__ __forceinline__ void head_split(const float *__restrict__ src,
+                                           const bf16x8 *__restrict__ w,
+                                           float bias, int chunks, int act,
+                                           float (*d)[kHeadPix],
+                                           float *s_out) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int t = wave; t < kHeadPix / 16; t += kHeadThreads / 64) {
+        const int p = t * 16 + (lane & 15);
+        const f32x4 *x = (const f32x4 *)(src + (size_t)(p < kP ? p : kP - 1) *
+                                                   chunks * 32) +
+                         (lane >> 4) * 2;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int c = 0; c < chunks; c++) {
+            const f32x4 lo = x[c * 8], hi = x[c * 8 + 1];
+            float v[8];
 #pragma unroll
-            for (int ky = 0; ky < 3; ky++)
+            for (int e = 0; e < 4; e++) {
+                v[e] = lo[e];
+                v[4 + e] = hi[e];
+            }
+            bf16x8 b[3], a[3];
+            split3(v, b);
 #pragma unroll
-                for (int kx = 0; kx < 3; kx++) {
-                    const float wv = s_w[c * 9 + ky * 3 + kx];
-                    acc0 += wv * pl[o0 + ky * SPs + kx];
-                    acc1 += wv * pl[o1 + ky * SPs + kx];
-                }
+            for (int q = 0; q < 3; q++) a[q] = w[(c * 3 + q) * 64 + lane];
+            acc = Op<__bf16>::mfma(a[0], b[2], acc);
+            acc = Op<__bf16>::mfma(a[2], b[0], acc);
+            acc = Op<__bf16>::mfma(a[1], b[1], acc);
+            acc = Op<__bf16>::mfma(a[0], b[1], acc);
+            acc = Op<__bf16>::mfma(a[1], b[0], acc);
+            acc = Op<__bf16>::mfma(a[0], b[0], acc);
         }
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if ((lane >> 4) * 4 + r < 9) d[(lane >> 4) * 4 + r][p] = acc[r];
     }
-    if (p0 < P) s_out[p0] = activate(acc0 + b, act);
-    if (p1 < P) s_out[p1] = activate(acc1 + b, act);
+    __syncthreads();
+    for (int p = tid; p < kP; p += kHeadThreads) {
+        const int y = p / kS, x = p % kS;
+        float v = 0.0f;
+#pragma unroll
+        for (int tap = 0; tap < 9; tap++) {
+            const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
+            if (yy >= 0 && yy < kS && xx >= 0 && xx < kS)
+                v += d[tap][yy * kS + xx];
+        }
+        s_out[p] = activate(v + bias, act);
+    }
     __syncthreads();
 }
 
@@ -204,53 +337,43 @@ __device__ float block_reduce(float v, bool is_max, float *s_red) {
     if (lane == 0) s_red[wave] = v;
     __syncthreads();
     float r = s_red[0];
-    for (int i = 1; i < kThreads / 64; i++)
+    for (int i = 1; i < kHeadThreads / 64; i++)
         r = is_max ? fmaxf(r, s_red[i]) : r + s_red[i];
     return r;
 }
 
-__global__ __launch_bounds__(kThreads) void policy_head_f32_kernel(
-    const float *__restrict__ in, const float *__restrict__ w,
+__global__ __launch_bounds__(kHeadThreads) void policy_head_f32_kernel(
+    const float *__restrict__ in, const bf16x8 *__restrict__ w,
     const float *__restrict__ b, float *__restrict__ raw,
-    float *__restrict__ out, int cin, int S, float temperature, int act) {
-    __shared__ float s_in[kHeadCK * kHeadSP * kHeadSP];
-    __shared__ float s_w[kHeadCK * 9];
-    __shared__ float s_logit[kMaxSide * kMaxSide];
-    __shared__ float s_red[kThreads / 64];
-    const int board = blockIdx.x, tid = threadIdx.x, P = S * S;
-    head_conv3(in + (size_t)board * cin * P, w, b[0], cin, S, act, s_in, s_w,
+    float *__restrict__ out, int chunks, float temperature, int act) {
+    __shared__ float d[9][kHeadPix];
+    __shared__ float s_logit[kP];
+    __shared__ float s_red[kHeadThreads / 64];
+    const int board = blockIdx.x, p = threadIdx.x;
+    head_split(in + (size_t)board * kP * chunks * 32, w, b[0], chunks, act, d,
                s_logit);
     // Network::softmax (Network.cpp:450-469): exp(x/T - max/T) / sum.
-    float mx = -INFINITY;
-    for (int p = tid; p < P; p += kThreads) mx = fmaxf(mx, s_logit[p]);
-    mx = block_reduce(mx, true, s_red);
-    const float alpha = mx / temperature;
-    float e[2] = {0.0f, 0.0f};
-    float sum = 0.0f;
-    for (int i = 0, p = tid; p < P; p += kThreads, i++) {
-        e[i] = expf(s_logit[p] / temperature - alpha);
-        sum += e[i];
-    }
-    sum = block_reduce(sum, false, s_red);
-    for (int i = 0, p = tid; p < P; p += kThreads, i++) {
-        if (raw) raw[(size_t)board * P + p] = s_logit[p];
-        if (out) out[(size_t)board * P + p] = e[i] / sum;
-    }
+    const float v = p < kP ? s_logit[p] : -INFINITY;
+    const float alpha = block_reduce(v, true, s_red) / temperature;
+    const float e = p < kP ? expf(v / temperature - alpha) : 0.0f;
+    const float sum = block_reduce(e, false, s_red);
+    if (p >= kP) return;
+    if (raw) raw[(size_t)board * kP + p] = v;
+    if (out) out[(size_t)board * kP + p] = e / sum;
 }
 
 // Last 1-channel conv + activation of the value net, written to h0
-// [n][S*S] for value_fc_head.
-__global__ __launch_bounds__(kThreads) void value_headconv_f32_kernel(
-    const float *__restrict__ in, const float *__restrict__ w,
-    const float *__restrict__ b, float *__restrict__ h0, int cin, int S,
+// [n][361] for value_fc_head.
+__global__ __launch_bounds__(kHeadThreads) void value_headconv_f32_kernel(
+    const float *__restrict__ in, const bf16x8 *__restrict__ w,
+    const float *__restrict__ b, float *__restrict__ h0, int chunks,
     int act) {
-    __shared__ float s_in[kHeadCK * kHeadSP * kHeadSP];
-    __shared__ float s_w[kHeadCK * 9];
-    __shared__ float s_h0[kMaxSide * kMaxSide];
-    const int board = blockIdx.x, tid = threadIdx.x, P = S * S;
-    head_conv3(in + (size_t)board * cin * P, w, b[0], cin, S, act, s_in, s_w,
+    __shared__ float d[9][kHeadPix];
+    __shared__ float s_h0[kP];
+    const int board = blockIdx.x, p = threadIdx.x;
+    head_split(in + (size_t)board * kP * chunks * 32, w, b[0], chunks, act, d,
                s_h0);
-    for (int p = tid; p < P; p += kThreads) h0[(size_t)board * P + p] = s_h0[p];
+    if (p < kP) h0[(size_t)board * kP + p] = s_h0[p];
 }
 
 // Batched inner-product head of the value net (Network.cpp:733-736):
@@ -312,17 +435,62 @@ __global__ __launch_bounds__(kThreads) void value_fc_kernel(
     }
 }
 
-template <int F, typename InT>
-hipError_t launch_conv(const void *in, const float *wpk, const float *bias,
-                       float *out, int n, int cin, int cout, int S,
-                       const ConvEpilogue &epi, hipStream_t stream) {
-    static_assert(ConvF32Cfg<F>::CK == (F == 5 ? 8 : 16),
-                  "chunk size must match f32_packed_k");
-    dim3 grid(n, (cout + kF32MBlock - 1) / kF32MBlock);
-    hipLaunchKernelGGL((conv_f32_kernel<F, InT>), grid, dim3(kThreads), 0,
-                       stream, static_cast<const InT *>(in), wpk, bias, out,
-                       cin, cout, S, epi);
+template <int F, int NB, int MTW, int NTW>
+hipError_t launch(const void *in, const uint16_t *wpk, const float *bias,
+                  float *out, int n, int cin, int cout,
+                  const ConvEpilogue &epi, hipStream_t stream) {
+    constexpr int BANDS = NTW == 6 ? 2 : 4;
+    const int mtiles = (cout + 15) / 16;
+    const dim3 grid(n * BANDS, (mtiles + 2 * MTW - 1) / (2 * MTW));
+    hipLaunchKernelGGL((conv_split<F, NB, MTW, NTW>), grid, dim3(kThreads), 0,
+                       stream, in, reinterpret_cast<const bf16x8 *>(wpk), bias,
+                       out, cin, f32_chunks(cin), cout, f32_stride(cout),
+                       mtiles, epi);
     return hipGetLastError();
+}
+
+// The piece of a conv that a workgroup takes, by a model of the time: a
+// workgroup costs its MFMAs (MTW x NTW) and its staging (2, or 4 for ten
+// rows), a CU's share is ceil(workgroups / 256) of them, and one workgroup
+// alone on a CU runs 1.6 times as long as its share of a full one. On a tie
+// the larger piece (it stages each input value for more outputs). The model
+// holds within 10% over n = 32 .. 256 (2.05 us a unit for 128 -> 128: 12
+// convs at n = 64 take 458 us with one m-tile and five rows a wave, 564 with
+// four; at n = 256 1339 us with four and ten, 1416 with four and five).
+template <int F, int NB>
+hipError_t launch_conv(const void *in, const uint16_t *wpk, const float *bias,
+                       float *out, int n, int cin, int cout,
+                       const ConvEpilogue &epi, hipStream_t stream) {
+    const int mtiles = (cout + 15) / 16;
+    int mtw = 4;
+    bool big = true;
+    double best = 0.0;
+    for (int k = 4; k >= 1; k--)
+        for (int rows10 = 1; rows10 >= 0; rows10--) {
+            const long long blocks = (mtiles + 2 * k - 1) / (2 * k);
+            const long long wgs = n * (rows10 ? 2LL : 4LL) * blocks;
+            const double q = (double)((wgs + 255) / 256);
+            const double t = (q < 2 ? 1.6 : q) *
+                             (k * (rows10 ? 6 : 3) + (rows10 ? 4 : 2));
+            if (best == 0.0 || t < best) {
+                best = t;
+                mtw = k;
+                big = rows10;
+            }
+        }
+    auto go = [&](auto m) {
+        constexpr int M = decltype(m)::value;
+        return big ? launch<F, NB, M, 6>(in, wpk, bias, out, n, cin, cout, epi,
+                                         stream)
+                   : launch<F, NB, M, 3>(in, wpk, bias, out, n, cin, cout, epi,
+                                         stream);
+    };
+    switch (mtw) {
+    case 1: return go(std::integral_constant<int, 1>());
+    case 2: return go(std::integral_constant<int, 2>());
+    case 3: return go(std::integral_constant<int, 3>());
+    default: return go(std::integral_constant<int, 4>());
+    }
 }
 
 bool act_ok(int act) {
@@ -332,42 +500,42 @@ bool act_ok(int act) {
 }  // namespace
 
 hipError_t conv_f32(int filter, bool u8_input, const void *in,
-                    const float *wpk, const float *bias, float *out, int n,
-                    int cin, int cout, int S, const ConvEpilogue &epi,
+                    const uint16_t *wpk, const float *bias, float *out, int n,
+                    int cin, int cout, const ConvEpilogue &epi,
                     hipStream_t stream) {
-    if (S < 1 || S > kMaxSide || n <= 0 || cin < 1 || cout < 1 ||
-        !act_ok(epi.act) || (epi.bn_mean && !epi.bn_inv_std))
+    if (n <= 0 || cin < 1 || cout < 1 || !act_ok(epi.act) ||
+        (epi.bn_mean && !epi.bn_inv_std))
         return hipErrorInvalidValue;
     if (filter == 3)
-        return u8_input ? launch_conv<3, uint8_t>(in, wpk, bias, out, n, cin,
-                                                  cout, S, epi, stream)
-                        : launch_conv<3, float>(in, wpk, bias, out, n, cin,
-                                                cout, S, epi, stream);
+        return u8_input ? launch_conv<3, 1>(in, wpk, bias, out, n, cin, cout,
+                                            epi, stream)
+                        : launch_conv<3, 3>(in, wpk, bias, out, n, cin, cout,
+                                            epi, stream);
     if (filter == 5)
-        return u8_input ? launch_conv<5, uint8_t>(in, wpk, bias, out, n, cin,
-                                                  cout, S, epi, stream)
-                        : launch_conv<5, float>(in, wpk, bias, out, n, cin,
-                                                cout, S, epi, stream);
+        return u8_input ? launch_conv<5, 1>(in, wpk, bias, out, n, cin, cout,
+                                            epi, stream)
+                        : launch_conv<5, 3>(in, wpk, bias, out, n, cin, cout,
+                                            epi, stream);
     return hipErrorInvalidValue;
 }
 
-hipError_t policy_head_f32(const float *in, const float *w, const float *b,
-                           float *raw, float *out, int n, int cin, int S,
+hipError_t policy_head_f32(const float *in, const uint16_t *w, const float *b,
+                           float *raw, float *out, int n, int cin,
                            float temperature, int act, hipStream_t stream) {
-    if (S < 1 || S > kMaxSide || n <= 0 || cin < 1 || !act_ok(act))
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(policy_head_f32_kernel, dim3(n), dim3(kThreads), 0,
-                       stream, in, w, b, raw, out, cin, S, temperature, act);
+    if (n <= 0 || cin < 1 || !act_ok(act)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(policy_head_f32_kernel, dim3(n), dim3(kHeadThreads), 0,
+                       stream, in, reinterpret_cast<const bf16x8 *>(w), b, raw,
+                       out, f32_chunks(cin), temperature, act);
     return hipGetLastError();
 }
 
-hipError_t value_headconv_f32(const float *in, const float *w,
+hipError_t value_headconv_f32(const float *in, const uint16_t *w,
                               const float *b, float *h0, int n, int cin,
-                              int S, int act, hipStream_t stream) {
-    if (S < 1 || S > kMaxSide || n <= 0 || cin < 1 || !act_ok(act))
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(value_headconv_f32_kernel, dim3(n), dim3(kThreads), 0,
-                       stream, in, w, b, h0, cin, S, act);
+                              int act, hipStream_t stream) {
+    if (n <= 0 || cin < 1 || !act_ok(act)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(value_headconv_f32_kernel, dim3(n), dim3(kHeadThreads),
+                       0, stream, in, reinterpret_cast<const bf16x8 *>(w), b,
+                       h0, f32_chunks(cin), act);
     return hipGetLastError();
 }
 

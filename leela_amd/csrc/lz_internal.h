@@ -12,17 +12,11 @@ namespace lz {
 constexpr int kMaxSide = 19;
 
 // ---- FP32 plain form (conv_fp32.hip) --------------------------------------
-// Output-channel block of one FP32 conv workgroup; packed weights are laid
-// out [cout/64][cin*k*k][64] with zero rows past cout.
-constexpr int kF32MBlock = 64;
-
-// K rows of a packed FP32 conv: the input channels are staged in chunks of
-// 8 (5x5) or 16 (3x3) channels, so cin is rounded up to whole chunks and
-// the extra rows are zero.
-__host__ __device__ inline int f32_packed_k(int filter, int cin) {
-    const int ck = filter == 5 ? 8 : 16;
-    return (cin + ck - 1) / ck * ck * filter * filter;
-}
+// Its convs run on BF16 MFMA with every FP32 value split into three BF16
+// parts. Input channels come in chunks of 32; activations between convs are
+// [n][361][f32_stride(C)], the channels past C zero.
+constexpr int f32_chunks(int cin) { return (cin + 31) / 32; }
+constexpr int f32_stride(int c) { return f32_chunks(c) * 32; }
 
 // Input planes per board the first conv may take (the reference's nets
 // take 32) and the widest trunk conv of the FP32 form.
@@ -40,20 +34,24 @@ struct ConvEpilogue {
     const float *bn_inv_std = nullptr;
 };
 
+// One same-padded conv over n 19x19 boards. in: byte planes [n][cin][361]
+// (u8_input) or activations; wpk: the three BF16 parts of the weights as MFMA
+// fragments, [chunk][tap][part][m-tile][lane][8].
 hipError_t conv_f32(int filter, bool u8_input, const void *in,
-                    const float *wpk, const float *bias, float *out, int n,
-                    int cin, int cout, int S, const ConvEpilogue &epi,
+                    const uint16_t *wpk, const float *bias, float *out, int n,
+                    int cin, int cout, const ConvEpilogue &epi,
                     hipStream_t stream);
 
-// Last 1-channel conv + activation + softmax(T): raw/out [n][S*S].
-hipError_t policy_head_f32(const float *in, const float *w, const float *b,
-                           float *raw, float *out, int n, int cin, int S,
+// Last 1-channel 3x3 conv + activation + softmax(T): raw/out [n][361]. w:
+// the parts of the nine taps' weights, [chunk][part][lane][8].
+hipError_t policy_head_f32(const float *in, const uint16_t *w, const float *b,
+                           float *raw, float *out, int n, int cin,
                            float temperature, int act, hipStream_t stream);
 
-// Last 1-channel conv + activation of the value net into h0 [n][S*S].
-hipError_t value_headconv_f32(const float *in, const float *w, const float *b,
-                              float *h0, int n, int cin, int S, int act,
-                              hipStream_t stream);
+// Last 1-channel conv + activation of the value net into h0 [n][361].
+hipError_t value_headconv_f32(const float *in, const uint16_t *w,
+                              const float *b, float *h0, int n, int cin,
+                              int act, hipStream_t stream);
 
 // Value inner-product head over a batch: FC (P -> hidden) + ELU, FC
 // (hidden -> 1), (1 + tanh) / 2. fc1_wt is the first FC transposed:

@@ -106,28 +106,18 @@ int upload_net(Net &net, int which, std::string *msg) {
     hipError_t e = hipSuccess;
     for (int k = 0; k < (int)net.layers.size() && e == hipSuccess; k++) {
         Layer &L = net.layers[k];
-        std::vector<float> packed;
-        if (L.kind == Layer::kConv && k < net.head) {
-            // [cout/64][Kp][64]: a workgroup's 64 output channels for one K
-            // row are contiguous, so the LDS copy is a straight stream; K
-            // rows past cin * k * k (a partial last chunk) stay zero.
-            const int K = L.cin * L.filter * L.filter;
-            const int Kp = f32_packed_k(L.filter, L.cin);
-            const int mbs = (L.cout + kF32MBlock - 1) / kF32MBlock;
-            packed.assign((size_t)mbs * Kp * kF32MBlock, 0.0f);
-            for (int o = 0; o < L.cout; o++)
-                for (int kk = 0; kk < K; kk++)
-                    packed[((size_t)(o / kF32MBlock) * Kp + kk) * kF32MBlock +
-                           o % kF32MBlock] = L.w[(size_t)o * K + kk];
-        } else if (L.kind == Layer::kFC && k == net.fc1) {
-            packed.assign(L.w.size(), 0.0f);
+        if (L.kind == Layer::kConv) {
+            e = upload(&L.d_w32,
+                       k < net.head ? pack_conv_split(L) : pack_head_split(L));
+        } else if (k == net.fc1) {
+            std::vector<float> t(L.w.size());
             for (int o = 0; o < L.cout; o++)
                 for (int i = 0; i < L.cin; i++)
-                    packed[(size_t)i * L.cout + o] = L.w[(size_t)o * L.cin + i];
+                    t[(size_t)i * L.cout + o] = L.w[(size_t)o * L.cin + i];
+            e = upload(&L.d_fc, t);
         } else {
-            packed = L.w;
+            e = upload(&L.d_fc, L.w);
         }
-        e = upload(&L.d_w32, packed);
         if (e == hipSuccess) e = upload(&L.d_b, L.b);
         if (e == hipSuccess && !L.bn_mean.empty()) {
             e = upload(&L.d_bn_mean, L.bn_mean);
@@ -172,9 +162,9 @@ int upload_net(Net &net, int which, std::string *msg) {
     A.c = c;
     A.m1 = L[0].cout;
     if (which == LZ_NET_VALUE) {
-        A.fc1_wt = L[net.fc1].d_w32;
+        A.fc1_wt = L[net.fc1].d_fc;
         A.fc1_b = L[net.fc1].d_b;
-        A.fc2_w = L[net.fc2].d_w32;
+        A.fc2_w = L[net.fc2].d_fc;
         A.fc2_b = L[net.fc2].d_b;
         A.hidden = L[net.fc1].cout;
     }
@@ -221,6 +211,60 @@ uint16_t float_to_bf16_rne(float f) {
         return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
+}
+
+namespace {
+
+float bf16_to_float(uint16_t h) {
+    const uint32_t u = (uint32_t)h << 16;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
+
+// The three BF16 parts of f (split3 in conv_fp32.hip).
+void split_bf16(float f, uint16_t part[3]) {
+    constexpr float kMax = 3.3895313892515355e38f;
+    part[0] = float_to_bf16_rne(std::isnan(f) ? f
+                                              : std::min(std::max(f, -kMax), kMax));
+    float r = f - bf16_to_float(part[0]);
+    part[1] = float_to_bf16_rne(r);
+    r -= bf16_to_float(part[1]);
+    part[2] = float_to_bf16_rne(r);
+}
+
+}  // namespace
+
+std::vector<uint16_t> pack_conv_split(const Layer &L) {
+    const int F = L.filter, cin = L.cin, cout = L.cout;
+    const int chunks = f32_chunks(cin), MT = (cout + 15) / 16;
+    std::vector<uint16_t> out((size_t)chunks * F * F * 3 * MT * 512, 0);
+    for (int o = 0; o < cout; o++)
+        for (int c = 0; c < cin; c++)
+            for (int tap = 0; tap < F * F; tap++) {
+                uint16_t part[3];
+                split_bf16(L.w[((size_t)o * cin + c) * F * F + tap], part);
+                const int lane = o % 16 + 16 * (c % 32 / 8);
+                for (int p = 0; p < 3; p++)
+                    out[((((size_t)(c / 32) * F * F + tap) * 3 + p) * MT +
+                         o / 16) * 512 + lane * 8 + c % 8] = part[p];
+            }
+    return out;
+}
+
+std::vector<uint16_t> pack_head_split(const Layer &L) {
+    const int cin = L.cin;
+    std::vector<uint16_t> out((size_t)f32_chunks(cin) * 3 * 512, 0);
+    for (int c = 0; c < cin; c++)
+        for (int tap = 0; tap < 9; tap++) {
+            uint16_t part[3];
+            split_bf16(L.w[(size_t)c * 9 + tap], part);
+            const int lane = tap + 16 * (c % 32 / 8);
+            for (int p = 0; p < 3; p++)
+                out[((size_t)(c / 32) * 3 + p) * 512 + lane * 8 + c % 8] =
+                    part[p];
+        }
+    return out;
 }
 
 uint16_t float_to_f16_rne(float f) {
@@ -309,6 +353,7 @@ std::vector<uint16_t> pack_conv_fragments(const Layer &L, FusedType type) {
 void free_net(Net &net) {
     for (auto &L : net.layers) {
         dfree(L.d_w32);
+        dfree(L.d_fc);
         dfree(L.d_b);
         dfree(L.d_wbf16);
         dfree(L.d_wf16);
@@ -317,7 +362,8 @@ void free_net(Net &net) {
         dfree(L.d_bn_mean);
         dfree(L.d_bn_inv_std);
         L.d_bn_mean = L.d_bn_inv_std = nullptr;
-        L.d_w32 = L.d_b = nullptr;
+        L.d_fc = L.d_b = nullptr;
+        L.d_w32 = nullptr;
         L.d_wbf16 = L.d_wf16 = nullptr;
         L.d_wf8 = nullptr;
         L.d_ws8 = nullptr;
@@ -335,6 +381,7 @@ int ensure_workspace(Workspace &ws, const Net nets[2], int n,
         if (!nets[k].layers.empty() && nets[k].layers[0].cin > cin0)
             cin0 = nets[k].layers[0].cin;
     }
+    ch = f32_stride(ch);
     const size_t P = (size_t)kMaxSide * kMaxSide;
     hipError_t e = dalloc(&ws.planes, (size_t)n * cin0 * P);
     if (e == hipSuccess) e = dalloc(&ws.act[0], (size_t)n * ch * P);
@@ -391,7 +438,6 @@ LaunchTimer::~LaunchTimer() {
 static int run_fp32(const Net &net, int which, int n, const uint8_t *planes,
                     float *raw, float *out, float temperature, Workspace &ws,
                     hipStream_t s, std::string *msg, LaunchTimer *timer) {
-    const int S = net.side;
     const void *x = planes;
     bool u8 = true;
     hipError_t e = timer ? timer->mark(s) : hipSuccess;
@@ -402,8 +448,8 @@ static int run_fp32(const Net &net, int which, int n, const uint8_t *planes,
         epi.act = L.act;
         epi.bn_mean = L.d_bn_mean;
         epi.bn_inv_std = L.d_bn_inv_std;
-        e = conv_f32(L.filter, u8, x, L.d_w32, L.d_b, y, n, L.cin, L.cout, S,
-                     epi, s);
+        e = conv_f32(L.filter, u8, x, L.d_w32, L.d_b, y, n, L.cin, L.cout, epi,
+                     s);
         if (e == hipSuccess && timer) e = timer->mark(s);
         x = y;
         u8 = false;
@@ -412,15 +458,16 @@ static int run_fp32(const Net &net, int which, int n, const uint8_t *planes,
     if (e == hipSuccess) {
         if (which == LZ_NET_POLICY) {
             e = policy_head_f32(static_cast<const float *>(x), H.d_w32, H.d_b,
-                                raw, out, n, H.cin, S, temperature, H.act, s);
+                                raw, out, n, H.cin, temperature, H.act, s);
         } else {
             const Layer &F1 = net.layers[net.fc1];
             const Layer &F2 = net.layers[net.fc2];
             e = value_headconv_f32(static_cast<const float *>(x), H.d_w32,
-                                   H.d_b, ws.h0, n, H.cin, S, H.act, s);
-            if (e == hipSuccess) e = value_fc_head(ws.h0, F1.d_w32, F1.d_b,
-                                                   F2.d_w32, F2.d_b, raw, out,
-                                                   n, S * S, F1.cout, s);
+                                   H.d_b, ws.h0, n, H.cin, H.act, s);
+            if (e == hipSuccess) e = value_fc_head(ws.h0, F1.d_fc, F1.d_b,
+                                                   F2.d_fc, F2.d_b, raw, out,
+                                                   n, net.side * net.side,
+                                                   F1.cout, s);
         }
         if (e == hipSuccess && timer) e = timer->mark(s);
     }

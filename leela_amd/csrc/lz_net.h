@@ -28,8 +28,9 @@ struct Layer {
     float *d_bn_mean = nullptr;
     float *d_bn_inv_std = nullptr;
     // Device copies.
-    float *d_w32 = nullptr;  // FP32: trunk packed [cout/64][K][64]; head conv
-                             // OIHW; FC1 transposed [in][out]; FC2 as is
+    uint16_t *d_w32 = nullptr;  // FP32 form's convs: three BF16 parts
+                                // (pack_conv_split / pack_head_split)
+    float *d_fc = nullptr;   // FC1 transposed [in][out]; FC2 as is
     float *d_b = nullptr;
     uint16_t *d_wbf16 = nullptr;  // BF16 MFMA fragments (fused kernels)
     uint16_t *d_wf16 = nullptr;   // FP16 MFMA fragments (fused kernels)
@@ -132,6 +133,14 @@ int run_net(const Net &net, int which, int precision, int n,
 // channel block, lane = row + 16 * g holding input channels
 // 32*cb + 8*g .. +7.
 std::vector<uint16_t> pack_conv_fragments(const Layer &L, FusedType type);
+
+// The FP32 form's weights: each value as three BF16 parts (round to nearest
+// even; the first part of a value past BF16's range is BF16's largest).
+// Trunk convs: [chunk of 32 inputs][tap][part][m-tile][lane][8], lane = row
+// + 16 * g holding input channels 8*g .. +7 of the chunk; the 3x3 head conv:
+// [chunk][part][lane][8], the taps as rows. Zero past cin, cout and tap 8.
+std::vector<uint16_t> pack_conv_split(const Layer &L);
+std::vector<uint16_t> pack_head_split(const Layer &L);
 
 // OCP e4m3 ("E4M3FN": bias 7, max 448, no infinities) with round to
 // nearest even; magnitudes beyond 448 saturate to 448.

@@ -1,0 +1,73 @@
+"""The FP32 form's convs (every value as three BF16 parts on BF16 MFMA)
+against the FP64 oracle, over the shapes and batch sizes where the kernel
+changes: channel counts around its blocks of 16 and chunks of 32, 5x5 and
+3x3 filters first and later, batches that take pieces of ten rows, five rows
+and few channels, byte planes that are not 0 / 1, weights of any scale.
+
+Bar: the parts hold FP32 values exactly and drop less than 2^-25 of a
+product, so a conv errs like an FP32 one: K^(1/2) roundings of 2^-24 on sums
+of K <= 5 * 5 * 160 terms, 4e-6 a layer at worst, six layers at most here:
+2e-5 of the largest logit.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (filter, cin, cout) of the trunk and head.
+NETS = {
+    "narrow": [(3, 5, 7), (5, 7, 17), (3, 17, 1)],
+    "odd": [(5, 22, 33), (3, 33, 48), (5, 48, 40), (3, 40, 1)],
+    "wide": [(3, 40, 160), (3, 160, 130), (3, 130, 96), (3, 96, 1)],
+    "reference_head": [(5, 32, 96), (3, 96, 128), (3, 128, 64), (3, 64, 1)],
+}
+
+
+def _table(name, scale):
+    rng = np.random.default_rng(len(name))
+    shapes = NETS[name]
+    table = []
+    for i, (f, cin, cout) in enumerate(shapes):
+        std = np.sqrt(2.0 / (cin * f * f))
+        # The first conv's weights carry `scale`, the last one's its inverse.
+        std *= scale if i == 0 else 1 / scale if i == len(shapes) - 1 else 1
+        w = rng.normal(0, std, (cout, cin, f, f)).astype(np.float32)
+        b = rng.normal(0, 0.1 * (scale if i < len(shapes) - 1 else 1),
+                       cout).astype(np.float32)
+        # ReLU keeps the scale from layer to layer.
+        act = 1 if cout > 1 else 2
+        table.append({"kind": "conv", "filter": f, "cin": cin, "cout": cout,
+                      "w": w, "b": b, "act": act, "bn": None})
+    return table
+
+
+@pytest.mark.parametrize("name,n,scale", [
+    ("narrow", 1, 1.0), ("narrow", 67, 1.0), ("odd", 1, 1.0),
+    ("odd", 33, 1.0), ("odd", 300, 1.0), ("wide", 2, 1.0), ("wide", 64, 1.0),
+    ("wide", 130, 1.0), ("reference_head", 96, 1.0),
+    ("reference_head", 257, 1.0), ("odd", 3, 1e30), ("odd", 3, 1e-25)])
+def test_fp32_form_matches_fp64(name, n, scale):
+    import leela_amd
+    import oracle
+    from leela_amd import caffe_weights as cw
+    from leela_amd import nets
+    print(f"case: {name} n={n} scale={scale}", flush=True)
+    table = _table(name, scale)
+    rng = np.random.default_rng(n)
+    planes = (rng.random((n, table[0]["cin"], 361)) < 0.3).astype(np.uint8)
+    planes[0] *= rng.integers(0, 256, planes[0].shape, dtype=np.uint8)
+    be = leela_amd.Backend(0)
+    try:
+        cw.push_layers(be, leela_amd.NET_POLICY, table)
+        be.load_net(leela_amd.NET_VALUE, nets.weight_set("A")[1])
+        be.finalize()
+        be.set_temperature(1.0)
+        raw, _ = be.forward(leela_amd.NET_POLICY, leela_amd.PREC_FP32, planes)
+    finally:
+        be.close()
+    oracle.load_blas()
+    want, _ = oracle.forward_f64(oracle.Net.from_table(table), planes,
+                                 oracle.HEAD_POLICY, temperature=1.0,
+                                 gemm=True)
+    for got, ref in zip(raw, want):  # (board 0 has inputs up to 255)
+        assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
