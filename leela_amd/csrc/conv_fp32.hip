@@ -378,48 +378,92 @@ __global__ __launch_bounds__(kHeadThreads) void value_headconv_f32_kernel(
 
 // Batched inner-product head of the value net (Network.cpp:733-736):
 // hidden = ELU(W1 h0 + b1), v = w2 . hidden + b2, out = (1 + tanh v) / 2.
-// A workgroup takes kFcBoards boards so every W1 element loaded from L2 is
-// used kFcBoards times; thread o accumulates output o for all of them. Four
-// boards per workgroup keeps a batch of 1024 on 256 workgroups (one per CU).
-constexpr int kFcBoards = 4;
+// A workgroup takes kFcBoards boards so that every W1 element from L2 is
+// used kFcBoards times. Bound: the latency of those reads (370 KB through
+// each CU). A lane forms four hidden units, the eight waves share the inputs
+// (every eighth each), and eight rows of W1 are on the way per wave: 64 KB
+// in flight on a CU, where a unit per thread had 8 KB: 22.6 / 22.8 -> 9.7 /
+// 10.9 us at 16 / 1024 boards (kernel trace). Four boards per workgroup keep a batch of 1024 on 256
+// workgroups (one per CU).
+constexpr int kFcBoards = 4, kFcThreads = 512;
 
-__global__ __launch_bounds__(kThreads) void value_fc_kernel(
+// VEC: H is a multiple of 4 (rows of W1 are read 16 bytes at a time).
+template <bool VEC>
+__global__ __launch_bounds__(kFcThreads) void value_fc_kernel(
     const float *__restrict__ h0, const float *__restrict__ w1t,
     const float *__restrict__ b1, const float *__restrict__ w2,
     const float *__restrict__ b2, float *__restrict__ raw,
     float *__restrict__ out, int n, int P, int H,
     const int *__restrict__ n_dev) {
-    __shared__ float s_h[kFcBoards][kMaxSide * kMaxSide];
-    __shared__ float s_red[kFcBoards][kThreads / 64];
+    constexpr int W = kFcThreads / 64;
+    __shared__ f32x4 s_h[kMaxSide * kMaxSide + 8 * W];  // [input] (boards)
+    __shared__ float s_part[W][kFcBoards][256];
+    __shared__ float s_red[kFcBoards][W];
     // A replayed graph sizes its grid for the bucket; the batch's board
     // count is then read from device memory.
     if (n_dev) n = min(n, *n_dev);
     const int b0 = blockIdx.x * kFcBoards, tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
     if (b0 >= n) return;
     const int nb = min(kFcBoards, n - b0);
-    for (int i = tid; i < kFcBoards * P; i += kThreads) {
-        const int bb = i / P, p = i % P;
-        s_h[bb][p] = bb < nb ? h0[(size_t)(b0 + bb) * P + p] : 0.0f;
+    for (int i = tid; i < P + 8 * W; i += kFcThreads) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int bb = 0; bb < kFcBoards; bb++)
+            if (bb < nb && i < P) v[bb] = h0[(size_t)(b0 + bb) * P + i];
+        s_h[i] = v;
     }
     __syncthreads();
     float part[kFcBoards];
 #pragma unroll
     for (int bb = 0; bb < kFcBoards; bb++) part[bb] = 0.0f;
-    for (int o = tid; o < H; o += kThreads) {
-        float acc[kFcBoards];
+    for (int j = 0; j < H; j += 256) {
+        const int o = j + lane * 4;
+        f32x4 acc[kFcBoards];
 #pragma unroll
-        for (int bb = 0; bb < kFcBoards; bb++) acc[bb] = 0.0f;
-#pragma unroll 8
-        for (int i = 0; i < P; i++) {
-            const float wv = w1t[(size_t)i * H + o];
+        for (int bb = 0; bb < kFcBoards; bb++) acc[bb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // Row i0 + u W of W1 (past the last input: the last row, times zeros).
+        f32x4 wv[8];
+        auto row_at = [&](int i) {
+            const float *row = w1t + (size_t)min(i, P - 1) * H;
+            f32x4 v;
+            if (VEC) {
+                v = *(const f32x4 *)(row + min(o, H - 4));
+            } else {
 #pragma unroll
-            for (int bb = 0; bb < kFcBoards; bb++) acc[bb] += wv * s_h[bb][i];
+                for (int r = 0; r < 4; r++) v[r] = row[min(o + r, H - 1)];
+            }
+            return v;
+        };
+#pragma unroll
+        for (int u = 0; u < 8; u++) wv[u] = row_at(wave + u * W);
+        for (int i0 = wave; i0 < P; i0 += 8 * W) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const f32x4 h = s_h[i0 + u * W], w = wv[u];
+                wv[u] = row_at(i0 + (u + 8) * W);
+#pragma unroll
+                for (int bb = 0; bb < kFcBoards; bb++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[bb][r] += w[r] * h[bb];
+            }
         }
-        const float bo = b1[o], wo = w2[o];
+        __syncthreads();
 #pragma unroll
-        for (int bb = 0; bb < kFcBoards; bb++) part[bb] += wo * elu(acc[bb] + bo);
+        for (int bb = 0; bb < kFcBoards; bb++)
+            *(f32x4 *)&s_part[wave][bb][lane * 4] = acc[bb];
+        __syncthreads();
+        if (tid < 256 && j + tid < H) {
+            const float bo = b1[j + tid], wo = w2[j + tid];
+#pragma unroll
+            for (int bb = 0; bb < kFcBoards; bb++) {
+                float v = s_part[0][bb][tid];
+#pragma unroll
+                for (int q = 1; q < W; q++) v += s_part[q][bb][tid];
+                part[bb] += wo * elu(v + bo);
+            }
+        }
     }
-    const int lane = tid & 63, wave = tid >> 6;
 #pragma unroll
     for (int bb = 0; bb < kFcBoards; bb++) {
         float v = part[bb];
@@ -429,7 +473,7 @@ __global__ __launch_bounds__(kThreads) void value_fc_kernel(
     __syncthreads();
     if (tid < nb) {
         float v = b2[0];
-        for (int w = 0; w < kThreads / 64; w++) v += s_red[tid][w];
+        for (int q = 0; q < W; q++) v += s_red[tid][q];
         if (raw) raw[b0 + tid] = v;
         if (out) out[b0 + tid] = (1.0f + tanhf(v)) / 2.0f;
     }
@@ -548,9 +592,10 @@ hipError_t value_fc_head(const float *h0, const float *fc1_wt,
     if (P < 1 || P > kMaxSide * kMaxSide || hidden < 1)
         return hipErrorInvalidValue;
     const int grid = (n + kFcBoards - 1) / kFcBoards;
-    hipLaunchKernelGGL(value_fc_kernel, dim3(grid), dim3(kThreads), 0, stream,
-                       h0, fc1_wt, fc1_b, fc2_w, fc2_b, raw, out, n, P,
-                       hidden, n_dev);
+    const auto fn =
+        hidden % 4 == 0 ? value_fc_kernel<true> : value_fc_kernel<false>;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(kFcThreads), 0, stream, h0, fc1_wt,
+                       fc1_b, fc2_w, fc2_b, raw, out, n, P, hidden, n_dev);
     return hipGetLastError();
 }
 

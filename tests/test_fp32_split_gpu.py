@@ -71,3 +71,44 @@ def test_fp32_form_matches_fp64(name, n, scale):
                                  gemm=True)
     for got, ref in zip(raw, want):  # (board 0 has inputs up to 255)
         assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("hidden,n", [(2, 1), (3, 5), (64, 2), (256, 4),
+                                      (258, 9), (300, 3), (513, 1)])
+def test_value_head_matches_fp64(hidden, n):
+    """The inner-product head at hidden sizes that are and are not multiples
+    of four or of the 256 units a pass holds, and batches that fill its
+    four-board workgroups or not. Sums of 361 and `hidden` products: FP32
+    roundings of 2^-24 * sqrt(361 * hidden) at most, 3e-5 of the result's
+    scale. (Not one unit: the oracle's first product then has no ELU, as the
+    reference's has none with one output.)"""
+    import leela_amd
+    import oracle
+    from leela_amd import nets
+    print(f"case: hidden={hidden} n={n}", flush=True)
+    rng = np.random.default_rng(hidden)
+
+    def layer(kind, f, cin, cout):
+        k = cin * max(f, 1) ** 2
+        w = rng.normal(0, np.sqrt(2.0 / k), cout * k).astype(np.float32)
+        w = w.reshape((cout, cin, f, f) if kind == nets.CONV else (cout, cin))
+        return (kind, f, cin, cout, w,
+                rng.normal(0, 0.1, cout).astype(np.float32))
+
+    val = [layer(nets.CONV, 3, 32, 16), layer(nets.CONV, 3, 16, 1),
+           layer(nets.FC, 0, 361, hidden), layer(nets.FC, 0, hidden, 1)]
+    planes = (rng.random((n, 32, 361)) < 0.3).astype(np.uint8)
+    be = leela_amd.Backend(0)
+    try:
+        be.load_net(leela_amd.NET_POLICY, nets.weight_set("A")[0])
+        be.load_net(leela_amd.NET_VALUE, val)
+        be.finalize()
+        raw, out = be.forward(leela_amd.NET_VALUE, leela_amd.PREC_FP32, planes)
+    finally:
+        be.close()
+    oracle.load_blas()
+    raw64, out64 = oracle.forward_f64(oracle.Net(val), planes,
+                                      oracle.HEAD_VALUE, gemm=True)
+    bar = 3e-5 * max(1.0, np.abs(raw64).max())
+    assert np.abs(raw.ravel() - raw64.ravel()).max() < bar
+    assert np.abs(out.ravel() - out64.ravel()).max() < bar
