@@ -32,15 +32,16 @@ hipError_t launch_playouts(const EncRecord *d_rec, int npos, int nplay,
 // Pattern playouts (mc_core.h's policy, the reference's) of n boards,
 // nplay each, playout j of board p seeded playout_seed(seed0 + p, j):
 // d_winrate[p] = mc_winrate for the side to move, NaN if one of its
-// playouts outgrew the device's candidate list. d_states holds nstates
-// playout states (a multiple of 64, pattern_state_bytes() each): the
-// persistent grid's threads. d_half_wins and d_overflow (n entries each)
-// are scratch.
+// playouts outgrew the device's candidate list. d_states holds the long
+// candidate lists of nstates wavefronts (pattern_state_bytes() each), the
+// most that run. d_next (one counter), d_half_wins and d_overflow (n entries
+// each) are scratch.
 size_t pattern_state_bytes();
 hipError_t launch_pattern_playouts(const EncRecord *d_rec, int npos,
                                    int nplay, uint32_t seed0,
                                    const mc::TablesView &tables,
                                    void *d_states, int nstates,
+                                   unsigned long long *d_next,
                                    uint32_t *d_half_wins,
                                    uint32_t *d_overflow, float *d_winrate,
                                    hipStream_t stream);

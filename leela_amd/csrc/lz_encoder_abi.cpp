@@ -45,16 +45,17 @@ struct lz_encoder {
     int next = 0;
     uint32_t *half_wins = nullptr;  // playout outcome counters, max_batch
     // Pattern playouts (allocated on first use): the policy's tables on the
-    // device, one playout state per thread of the persistent grid, the
-    // per-position counters of abandoned playouts, and the event after the
-    // last launch that used them (the next launch waits for it, whatever
-    // its stream).
+    // device, the long candidate lists of the persistent grid's wavefronts,
+    // its work counter, the per-position counters of abandoned playouts, and
+    // the event after the last launch that used them (the next launch waits
+    // for it, whatever its stream).
     int32_t *pat_g = nullptr;
     uint16_t *pat_index[2] = {nullptr, nullptr};
     float *pat_fw = nullptr;
     float *pat_pw = nullptr;
     void *pat_states = nullptr;
     int pat_nstates = 0;
+    unsigned long long *pat_next = nullptr;
     uint32_t *pat_overflow = nullptr;
     hipEvent_t pat_done = nullptr;
     bool pat_used = false;
@@ -135,7 +136,7 @@ void lz_encoder_destroy(lz_encoder *e) {
     for (void *p : {(void *)e->half_wins, (void *)e->pat_g,
                     (void *)e->pat_index[0], (void *)e->pat_index[1],
                     (void *)e->pat_fw, (void *)e->pat_pw, e->pat_states,
-                    (void *)e->pat_overflow})
+                    (void *)e->pat_overflow, (void *)e->pat_next})
         if (p) (void)hipFree(p);
     delete e;
 }
@@ -236,12 +237,10 @@ int playouts(lz_encoder *e, const lz_position *const *pos, int n, int nplay,
     return release_slot(e, sl, s);
 }
 
-// Threads of the pattern playouts' persistent grid: 3,072 wavefronts (12
-// per CU of the part, the kernel's occupancy), each thread with its own
-// playout state (~23 KB: 4.5 GB in all). The playouts are latency-bound
-// pointer chasing, so resident wavefronts are what sets the rate: a third
-// of this grid ran 19x19 playouts 1.4x slower.
-constexpr int kPatternThreads = 196608;
+// Wavefronts of the pattern playouts' persistent grid: 20 on each CU, what
+// their registers and LDS allow. Each has a long candidate list in global
+// memory (16 KB: 81 MB in all).
+constexpr int kPatternWaves = 256 * 20;
 
 template <typename T>
 hipError_t upload(T **dst, const std::vector<T> &v) {
@@ -270,15 +269,18 @@ int pattern_setup(lz_encoder *e) {
     if (err == hipSuccess)
         err = hipEventCreateWithFlags(&e->pat_done, hipEventDisableTiming);
     if (err == hipSuccess)
+        err = hipMalloc(reinterpret_cast<void **>(&e->pat_next),
+                        sizeof(unsigned long long));
+    if (err == hipSuccess)
         err = hipMalloc(&e->pat_states,
-                        lz::pattern_state_bytes() * (size_t)kPatternThreads);
+                        lz::pattern_state_bytes() * (size_t)kPatternWaves);
     if (err != hipSuccess) {
         if (e->pat_states) (void)hipFree(e->pat_states);
         e->pat_states = nullptr;
         return e->fail(LZ_ERR_NOMEM, "pattern playout setup: %s",
                        hipGetErrorString(err));
     }
-    e->pat_nstates = kPatternThreads;
+    e->pat_nstates = kPatternWaves;
     return LZ_OK;
 }
 
@@ -310,7 +312,7 @@ int pattern_playouts(lz_encoder *e, const lz_position *const *pos, int n,
     tv.pattern_weight = e->pat_pw;
     hipError_t err = lz::launch_pattern_playouts(
         sl->dev, n, nplay, seed0, tv, e->pat_states, e->pat_nstates,
-        e->half_wins, e->pat_overflow, d_winrate, s);
+        e->pat_next, e->half_wins, e->pat_overflow, d_winrate, s);
     if (err == hipSuccess) err = hipEventRecord(e->pat_done, s);
     if (err != hipSuccess)
         return e->fail(LZ_ERR_HIP, "pattern playout launch: %s",

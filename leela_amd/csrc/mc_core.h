@@ -103,8 +103,9 @@ struct MoveList {
     }
     LZ_HD bool empty() const { return n == 0; }
     LZ_HD int size() const { return n; }
-    LZ_HD Move &back() { return m[n - 1]; }
-    LZ_HD Move &operator[](int i) { return m[i]; }
+    LZ_HD Move get(int i) const { return m[i]; }
+    LZ_HD void set(int i, const Move &x) { m[i] = x; }
+    LZ_HD void add_back(int flag, const TablesView &t) { m[n - 1].add(flag, t); }
     LZ_HD void push(int v, int flag, const TablesView &t) {
         if (n >= CAP) {
             overflow = true;
@@ -114,6 +115,23 @@ struct MoveList {
         x.word = (uint32_t)(v + 1) << 22;
         x.score = 1.0f;
         x.add(flag, t);
+    }
+};
+
+// How a playout runs its independent steps: the host one after another; the
+// device's form (mc_playout.hip) spreads them over a wavefront's lanes.
+struct SerialExec {
+    // The first i of 0 .. n - 1 for which f(i), or -1.
+    template <class F>
+    LZ_HD static int first(int n, F f) {
+        for (int i = 0; i < n; i++)
+            if (f(i)) return i;
+        return -1;
+    }
+    // f(i) for every i of 0 .. n - 1.
+    template <class F>
+    LZ_HD static void each(int n, F f) {
+        for (int i = 0; i < n; i++) f(i);
     }
 };
 
@@ -262,13 +280,14 @@ public:
     LZ_HD bool is_eye(int color, int v) const {
         if (!(nbr_[v] & (4 << (4 * color)))) return false;
         const int W = size_ + 2;
-        int cnt[4] = {0, 0, 0, 0};
-        cnt[sq_[v - 1 - W]]++;
-        cnt[sq_[v + 1 - W]]++;
-        cnt[sq_[v - 1 + W]]++;
-        cnt[sq_[v + 1 + W]]++;
-        if (cnt[kInval] == 0) return cnt[1 - color] <= 1;
-        return cnt[1 - color] == 0;
+        const int diag[4] = {v - 1 - W, v + 1 - W, v - 1 + W, v + 1 + W};
+        int enemy = 0, off = 0;
+        for (int i = 0; i < 4; i++) {
+            const int c = sq_[diag[i]];
+            enemy += c == 1 - color;
+            off += c == kInval;
+        }
+        return off == 0 ? enemy <= 1 : enemy == 0;
     }
     LZ_HD bool no_eye_fill(int v, int to_move) const {
         return !is_eye(to_move, v);
@@ -284,7 +303,9 @@ public:
         return true;
     }
 
-    LZ_HD bool is_suicide(int v, int color) {
+    // FastBoard::is_suicide without its trial stone: with it, every string
+    // next to v (each counted once) has one liberty less.
+    LZ_HD bool is_suicide(int v, int color) const {
         if (count(kEmpty, v)) return false;
         bool connecting = false;
         for (int k = 0; k < 4; k++) {
@@ -297,17 +318,15 @@ public:
                 return false;  // captures
             }
         }
-        add_neighbour(v, color);
         bool opps_live = true, ours_die = true;
         for (int k = 0; k < 4; k++) {
             const int ai = v + dirs_[k];
-            const int libs = libs_at(ai);
+            const int libs = libs_at(ai) - 1;
             if (libs == 0 && sq_[ai] != color)
                 opps_live = false;
             else if (libs != 0 && sq_[ai] == color)
                 ours_die = false;
         }
-        remove_neighbour(v, color);
         return connecting ? (opps_live && ours_die) : opps_live;
     }
 
@@ -395,8 +414,8 @@ public:
                                           : kSaving3P,
                        t);
                 const int libs = count(kEmpty, atari);
-                if (libs == 2) m.back().add(kSaving2Lib, t);
-                if (libs == 3) m.back().add(kSaving3Lib, t);
+                if (libs == 2) m.add_back(kSaving2Lib, t);
+                if (libs == 3) m.add_back(kSaving3Lib, t);
             }
             const bool sa = self_atari(color, atari);
             const bool kill = kill_neighbours(ai, komove, m, t);
@@ -461,32 +480,28 @@ private:
     LZ_HD int libs_at(int v) const { return libs_[parent_[v]]; }
 
     LZ_HD void add_neighbour(int v, int color) {
-        int pars[4], cnt = 0;
+        int pars[4];
         for (int k = 0; k < 4; k++) {
             const int ai = v + dirs_[k];
             nbr_[ai] = (uint16_t)(nbr_[ai] + (1 << (4 * color)) - (1 << 8));
             const int p = parent_[ai];
             bool found = false;
-            for (int i = 0; i < cnt; i++) found |= pars[i] == p;
-            if (!found) {
-                libs_[p]--;
-                pars[cnt++] = p;
-            }
+            for (int i = 0; i < k; i++) found |= pars[i] == p;
+            pars[k] = p;
+            if (!found) libs_[p]--;
         }
     }
 
     LZ_HD void remove_neighbour(int v, int color) {
-        int pars[4], cnt = 0;
+        int pars[4];
         for (int k = 0; k < 4; k++) {
             const int ai = v + dirs_[k];
             nbr_[ai] = (uint16_t)(nbr_[ai] + (1 << 8) - (1 << (4 * color)));
             const int p = parent_[ai];
             bool found = false;
-            for (int i = 0; i < cnt; i++) found |= pars[i] == p;
-            if (!found) {
-                libs_[p]++;
-                pars[cnt++] = p;
-            }
+            for (int i = 0; i < k; i++) found |= pars[i] == p;
+            pars[k] = p;
+            if (!found) libs_[p]++;
         }
     }
 
@@ -603,11 +618,11 @@ private:
                         if (atari != komove) {
                             m.push(atari, capture_flag(stones_[par]), t);
                             const int sav = string_size(v);
-                            m.back().add(sav == 1   ? kSaving1
-                                         : sav == 2 ? kSaving2
-                                                    : kSaving3P,
-                                         t);
-                            m.back().add(kSavingKill, t);
+                            m.add_back(sav == 1   ? kSaving1
+                                       : sav == 2 ? kSaving2
+                                                  : kSaving3P,
+                                       t);
+                            m.add_back(kSavingKill, t);
                         }
                         seen[nseen++] = par;
                     }
@@ -812,9 +827,9 @@ private:
     int ncritical_ = 0;
 };
 
-// FastState's playout state around a PlayBoard; CAP is the capacity of
-// the move generator's candidate list.
-template <int CAP>
+// FastState's playout state around a PlayBoard; Moves is the move generator's
+// candidate list, Exec how independent steps run.
+template <class Moves, class Exec>
 struct PlayStateT {
     PlayBoard board;
     int to_move = kBlack;
@@ -824,8 +839,8 @@ struct PlayStateT {
     int passes = 0;
     int movenum = 0;
     float komi = 7.5f;
-    bool overflow = false;   // a candidate list outgrew CAP: abandoned
-    MoveList<CAP> moves;     // scratch of the move generator
+    bool overflow = false;   // the candidate list overflowed: abandoned
+    Moves moves;             // scratch of the move generator
 
     // FastState::play_move_fast.
     LZ_HD int play_fast(int v) {
@@ -852,21 +867,17 @@ struct PlayStateT {
         const int dir = (int)rng.randfix<2>();
         const int n = board.empty_count();
         const int start = (int)rng.randuint16((uint16_t)n);
-        if (dir == 0) {
-            for (int i = start; i < n; i++)
-                if (try_move(color, board.empty_at(i))) return board.empty_at(i);
-            for (int i = 0; i < start; i++)
-                if (try_move(color, board.empty_at(i))) return board.empty_at(i);
-        } else {
-            for (int i = start; i >= 0; i--)
-                if (try_move(color, board.empty_at(i))) return board.empty_at(i);
-            for (int i = n - 1; i > start; i--)
-                if (try_move(color, board.empty_at(i))) return board.empty_at(i);
-        }
-        return kPassMove;
+        // The list from `start` on, up (dir 0) or down, around its end.
+        auto at = [&](int k) {
+            int i = dir == 0 ? start + k : start - k;
+            i = i >= n ? i - n : i < 0 ? i + n : i;
+            return board.empty_at(i);
+        };
+        const int k = Exec::first(n, [&](int i) { return try_move(color, at(i)); });
+        return k < 0 ? kPassMove : at(k);
     }
 
-    LZ_HD void flag_move(Move &m, int color, const TablesView &t) {
+    LZ_HD void flag_move(Move &m, int color, const TablesView &t) const {
         m.score *= t.pattern_weight[pattern_index(
             t, color, board.pattern_augment(m.sq()))];
         if (!board.self_atari(color, m.sq())) return;
@@ -884,6 +895,17 @@ struct PlayStateT {
         if (m.has(kPattern)) m.add(kPatternSA, t);
         if (m.has(kSaving1) || m.has(kSaving2) || m.has(kSaving3P))
             m.add(kSavingSA, t);
+    }
+
+    // flag_move for the candidates from i0 on (but the pass); each only reads
+    // the board.
+    LZ_HD void flag_moves(int i0, int color, const TablesView &t) {
+        Exec::each(moves.size() - i0, [&](int k) {
+            Move m = moves.get(i0 + k);
+            if (m.sq() == kPassMove) return;
+            flag_move(m, color, t);
+            moves.set(i0 + k, m);
+        });
     }
 
     // FastState::play_random_move (FastState.cpp:168-255): plays and
@@ -906,10 +928,11 @@ struct PlayStateT {
         }
         if (moves.overflow) return abandon();
         float cumul = 0.0f, best = 0.0f;
+        flag_moves(0, color, t);
         for (int i = 0; i < moves.size(); i++) {
-            flag_move(moves[i], color, t);
-            cumul += moves[i].score;
-            if (moves[i].score > best) best = moves[i].score;
+            const float score = moves.get(i).score;
+            cumul += score;
+            if (score > best) best = score;
         }
         // No good move yet: random moves from the empty list, and a pass.
         if (moves.empty() || best < kBound) {
@@ -921,10 +944,9 @@ struct PlayStateT {
             }
             moves.push(kPassMove, kPass, t);
             if (moves.overflow) return abandon();
-            for (int i = scored; i < moves.size(); i++) {
-                if (moves[i].sq() != kPassMove) flag_move(moves[i], color, t);
-                cumul += moves[i].score;
-            }
+            flag_moves(scored, color, t);
+            for (int i = scored; i < moves.size(); i++)
+                cumul += moves.get(i).score;
         }
         // The draw: the first move whose running sum of scores reaches
         // index (the running sums are formed again in the same order, so
@@ -932,8 +954,9 @@ struct PlayStateT {
         const float index = rng.randflt() * cumul;
         float run = 0.0f;
         for (int i = 0; i < moves.size(); i++) {
-            run += moves[i].score;
-            if (index <= run) return play_fast(moves[i].sq());
+            const Move m = moves.get(i);
+            run += m.score;
+            if (index <= run) return play_fast(m.sq());
         }
         return play_fast(kPassMove);
     }
@@ -958,11 +981,10 @@ struct PlayStateT {
 };
 
 // The host's state: a candidate list no position can outgrow.
-using PlayState = PlayStateT<kMaxMoves>;
-// The device's state (one per thread of the persistent grid, ~23 KB): a
-// list of 2,048 candidates, and an abandoned playout beyond that.
+using PlayState = PlayStateT<MoveList<kMaxMoves>, SerialExec>;
+// The device's list holds 2,048 candidates; a playout beyond that is
+// abandoned.
 constexpr int kDevMoves = 2048;
-using DevPlayState = PlayStateT<kDevMoves>;
 
 }  // namespace mc
 }  // namespace lz

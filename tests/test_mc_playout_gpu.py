@@ -1,5 +1,5 @@
 """The reference's pattern playout policy on the GPU (mc_playout.hip: one
-playout per thread, the host's source, mc_core.h). Pinned to the host
+playout per wavefront, the host's source, mc_core.h). Pinned to the host
 playouts bit for bit (same positions, same seeds: equal win rates), and to
 the reference itself through the golden playouts: the device win rate of a
 golden position equals the mean outcome of the reference's own playouts
@@ -48,6 +48,20 @@ def test_device_pattern_playouts_equal_host(enc):
                    for i, p in enumerate(pos)], np.float32)
     np.testing.assert_array_equal(dl, hl)
     assert (dev != dl).any()
+
+
+@pytest.mark.parametrize("npos,nplay,side", [(1, 1, 9), (3, 7, 5), (1, 63, 13),
+                                             (1, 5121, 9), (2, 2561, 7)])
+def test_device_pattern_playouts_at_the_grid_edges(enc, npos, nplay, side):
+    """One playout, fewer than a CU holds, and one or two more than the grid's
+    5120 wavefronts: every playout is played once."""
+    print(f"case: {npos} x {nplay} on {side}x{side}", flush=True)
+    pos = [Position.random(600 + i, side, side * side // 2)
+           for i in range(npos)]
+    dev = enc.playout_winrates(PositionBatch(pos), nplay, 31, PLAYOUT_PATTERN)
+    host = np.array([p.playout_winrate(nplay, 31 + i, PLAYOUT_PATTERN)
+                     for i, p in enumerate(pos)], np.float32)
+    np.testing.assert_array_equal(dev, host)
 
 
 def test_device_pattern_playouts_match_reference_golden(enc):
