@@ -1,5 +1,5 @@
 // encoder.hip — the nets' input planes computed on the GPU, one wavefront
-// per board.
+// per board or, in small batches, per quarter of a board's points.
 //
 // Reference: Network::gather_features_policy / gather_features_value
 // (Network.cpp:883-1201) and the FastBoard queries behind them: string
@@ -510,13 +510,23 @@ __device__ __forceinline__ PlaneMap plane_map(int net) {
 
 constexpr int kTaskLose = 1 << 20;
 
+// A board is `parts` workgroups of one wavefront; part w of them takes the
+// output rows w, w + parts, ...: their points' after-liberties, ladder tasks
+// and plane bytes (a point's tasks decide its own planes only). The strings
+// each part finds for itself.
 __global__ __launch_bounds__(64) void encode_kernel(const EncRecord *recs,
+                                                    int n, int parts,
                                                     int symmetry,
                                                     uint8_t *out_policy,
                                                     uint8_t *out_value,
                                                     uint64_t *ovf) {
     const int lane = threadIdx.x;
-    const EncRecord &r = recs[blockIdx.x];
+    // A board's parts lie eight blocks apart: on one XCD, whose L2 then
+    // joins their bytes into whole lines.
+    const int part = (int)blockIdx.x / 8 % parts;
+    const int board = (int)blockIdx.x / (8 * parts) * 8 + (int)blockIdx.x % 8;
+    if (board >= n) return;
+    const EncRecord &r = recs[board];
     const int side = r.side, W = side + 2, G = W * W, P = side * side;
     const int tm = r.to_move, opp = tm ^ 1;
 
@@ -531,7 +541,7 @@ __global__ __launch_bounds__(64) void encode_kernel(const EncRecord *recs,
     }
     if (lane == 0) {
         s_ntasks = 0;
-        s_ovf = ovf + (size_t)blockIdx.x * kStrOvf * kWords;
+        s_ovf = ovf + (size_t)board * kStrOvf * kWords;
     }
     __syncthreads();
     const int d[4] = {-W, 1, W, -1};  // FastBoard::m_dirs order
@@ -547,7 +557,21 @@ __global__ __launch_bounds__(64) void encode_kernel(const EncRecord *recs,
     const Bits E = bits_andnot(on, bits_or(stones[0], stones[1]));
 
     // 2. String ids (representatives in vertex order), the stones of every
-    // string, then its liberty count.
+    // string, then its liberty count. The overflow area is one per board: a
+    // board that needs it is left to its first part as a whole.
+    if (parts > 1) {
+        int heads = 0;
+        for (int v0 = 0; v0 < G; v0 += 64) {
+            const int v = v0 + lane;
+            const int c = v < G ? s_sq[v] : kOff;
+            heads += __popcll(__ballot((c == kBlack || c == kWhite) &&
+                                       s_head[v] == v));
+        }
+        if (heads > kStrCap) {
+            if (part > 0) return;
+            parts = 1;
+        }
+    }
     {
         int base = 0;
         for (int v0 = 0; v0 < G; v0 += 64) {
@@ -594,8 +618,19 @@ __global__ __launch_bounds__(64) void encode_kernel(const EncRecord *recs,
     }
     __syncthreads();
 
+    // This part's output points: k-th of its rows' points.
+    const int rows = (side - part + parts - 1) / parts, mine = rows * side;
+    auto out_index = [&](int k) {
+        return (part + k / side * parts) * side + k % side;
+    };
+    auto vertex = [&](int i) {
+        const int src = rotate_idx(i, symmetry, side);
+        return (src / side + 1) * W + src % side + 1;
+    };
+
     // 3. Lane per empty point: after-liberties and ladder tasks.
-    for (int v = lane; v < G; v += 64) {
+    for (int k = lane; k < mine; k += 64) {
+        const int v = vertex(out_index(k));
         if (s_sq[v] != kEmpty) continue;
         int nh[4], ncol[4];
 #pragma unroll
@@ -740,10 +775,10 @@ __global__ __launch_bounds__(64) void encode_kernel(const EncRecord *recs,
 
     // 5. Lane per output index: the plane bytes of the rotated point, for
     // each net asked for.
-    for (int i = lane; i < P; i += 64) {
-        const int src = rotate_idx(i, symmetry, side);
-        const int x = src % side, y = src / side;
-        const int v = (y + 1) * W + (x + 1);
+    for (int k = lane; k < mine; k += 64) {
+        const int i = out_index(k);
+        const int v = vertex(i);
+        const int x = v % W - 1, y = v / W - 1;
         const int c = s_sq[v];
         const bool line3 = x == 2 || x == side - 3 || y == 2 || y == side - 3;
         const int libs = c == kEmpty ? 0 : s_libs[s_head[v]];
@@ -786,8 +821,16 @@ hipError_t launch_encode(const EncRecord *d_rec, int n, int symmetry,
                          hipStream_t stream) {
     if (n <= 0 || (!d_policy && !d_value)) return hipSuccess;
     if (!d_ovf) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(encode_kernel, dim3(n), dim3(64), 0, stream, d_rec,
-                       symmetry, d_policy, d_value, d_ovf);
+    // Up to 1024 boards in four parts: a launch lasts as long as its slowest
+    // wavefront, whose ladder readings take turns where they part, and the
+    // chip holds 2048 of these wavefronts. One part against four, us: 111 /
+    // 70 at 1 board, 266 / 148 at 16, 394 / 298 at 256, 525 / 485 at 1024;
+    // at 2048 536 / 564 and at 4096 748 / 914, where the parts' own string
+    // finding only adds to a full chip.
+    const int parts = n <= 1024 ? 4 : 1;
+    hipLaunchKernelGGL(encode_kernel, dim3((n + 7) / 8 * 8 * parts), dim3(64),
+                       0, stream, d_rec, n, parts, symmetry, d_policy, d_value,
+                       d_ovf);
     return hipGetLastError();
 }
 

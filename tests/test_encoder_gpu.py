@@ -13,6 +13,7 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+from leela_amd import positions
 from leela_amd.backend import LeelaError
 from leela_amd.positions import (NET_POLICY, NET_VALUE, DeviceEncoder,
                                  Position, encode_batch)
@@ -151,3 +152,27 @@ def test_many_strings_overflow_matches_host(enc):
         got = enc.encode(pos, net).cpu().numpy()
         want = encode_batch(pos, net, 0, 8)
         assert np.array_equal(got.reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("n,side", [(1, 5), (7, 9), (9, 13), (1024, 19),
+                                    (1025, 9)])
+def test_device_encoder_at_the_edges_of_its_parts(n, side):
+    """Batches of up to 1024 boards are encoded in four parts a board, in
+    blocks of eight boards, larger ones in one: every byte of both nets'
+    planes equals the host encoder's, and nothing past them is written."""
+    import torch
+    print(f"case: {n} boards of {side}", flush=True)
+    pos = [positions.Position.random(700 + i, side, side * side * 2 // 3)
+           for i in range(n)]
+    enc = positions.DeviceEncoder(0, max_batch=n)
+    k = n * 32 * side * side
+    out = [torch.full((k + 64,), 7, dtype=torch.uint8, device="cuda:0")
+           for _ in range(2)]
+    enc.encode_both_into(pos, out[0].data_ptr(), out[1].data_ptr(), 5,
+                         torch.cuda.current_stream().cuda_stream)
+    for net, o in enumerate(out):
+        got = o.cpu().numpy()
+        want = positions.encode_batch(pos, net, 5)
+        np.testing.assert_array_equal(got[:k], want.ravel())
+        assert (got[k:] == 7).all()
+    enc.close()
