@@ -102,6 +102,8 @@ int lz_finalize(lz_ctx *ctx);
  * over several workgroups, instead of one workgroup per board running the
  * whole chain. Same outputs bit for bit; lower latency for small batches
  * (the leaf queue's smallest bucket, synchronous single-position calls).
+ * With the default, policy batches of up to 96 boards, and up to 96 boards
+ * past whole multiples of the CU count of larger ones, run so too.
  * 0 keeps every batch on the persistent kernel. Launch-shape setting with
  * no reference counterpart; applies to forwards and queue graphs captured
  * after the call. */

@@ -1015,11 +1015,11 @@ hipError_t layered_run(int which, const uint8_t *planes, const FusedArgs &a,
     // Two policy tiles per board, then two value tiles: each net keeps its
     // own layout's zero halos.
     T *pol = static_cast<T *>(tiles);
-    T *val = pol + 2 * (size_t)kLayeredMaxBoards * ltile<144>();
+    T *val = pol + 2 * (size_t)kLayeredTailBoards * ltile<144>();
     T *buf[2];
     if (which == 0) {
         buf[0] = pol;
-        buf[1] = pol + (size_t)kLayeredMaxBoards * ltile<144>();
+        buf[1] = pol + (size_t)kLayeredTailBoards * ltile<144>();
     } else {
         buf[0] = val;
         buf[1] = val + (size_t)kLayeredMaxBoards * ltile<80>();
@@ -1082,7 +1082,8 @@ int fused_blocks_per_cu(int which, int wm) {
 int ragged_slot_capacity(int side) { return slot_capacity(side); }
 
 size_t layered_tile_bytes() {
-    return 2 * (size_t)kLayeredMaxBoards * (ltile<144>() + ltile<80>()) *
+    return 2 * ((size_t)kLayeredTailBoards * ltile<144>() +
+                (size_t)kLayeredMaxBoards * ltile<80>()) *
            sizeof(uint16_t);
 }
 
@@ -1092,7 +1093,8 @@ hipError_t fused_forward_layered(int which, FusedType type,
                                  float temperature, void *tiles,
                                  hipStream_t stream, const uint32_t *bits) {
     if (n <= 0) return hipSuccess;
-    if (n > kLayeredMaxBoards || !tiles || args.slots ||
+    if (n > (which == 0 ? kLayeredTailBoards : kLayeredMaxBoards) || !tiles ||
+        args.slots ||
         type == FusedType::kFP8)
         return hipErrorInvalidValue;
     return type == FusedType::kBF16

@@ -79,12 +79,16 @@ hipError_t fused_forward(int which, FusedType type, const uint8_t *planes,
                          hipStream_t stream);
 
 // Layered form of fused_forward for at most kLayeredMaxBoards 19x19 boards
+// (policy: kLayeredTailBoards)
 // (BF16 / FP16, not ragged): one launch per conv, each conv of a board
 // split over several workgroups, activations between convs in `tiles`
 // (layered_tile_bytes(), zeroed once before first use: the tiles' halos
 // must stay zero). Bitwise the same outputs as fused_forward, at a lower
 // latency for small batches.
+// (kLayeredTailBoards: the most it takes as the rest of a larger policy
+// batch, see run_net.)
 constexpr int kLayeredMaxBoards = 64;
+constexpr int kLayeredTailBoards = 96;
 size_t layered_tile_bytes();
 // bits (optional): the same boards' planes packed one 32-bit word per
 // point, bit c = plane c ([n][361]), which the stem reads instead of the

@@ -535,14 +535,42 @@ int run_net(const Net &net, int which, int precision, int n,
         const FusedType ft = bf ? FusedType::kBF16 : FusedType::kFP16;
         if (e == hipSuccess) {
             // (The layered stem copies planes 16 bytes at a time.)
-            if (!ragged && ws.tiles && n <= net.layered_max &&
-                reinterpret_cast<uintptr_t>(d_planes) % 16 == 0)
+            const bool layered =
+                !ragged && ws.tiles && net.layered_max > 0 &&
+                reinterpret_cast<uintptr_t>(d_planes) % 16 == 0;
+            // The persistent policy kernel takes a pass of the chip (a board
+            // per CU) as long for a few boards as for all: 205 us up to 200
+            // boards, 190 more for any second pass. The layered form takes
+            // 155 us for 64 and 172 for 96, so batches of that size, and the
+            // boards past whole passes of larger ones, run in it (same
+            // bits): 257 boards 426 -> 335 us, 331 435 -> 399, 352 439 ->
+            // 417, 600 680 -> 653. The value net's passes are of 512 boards
+            // and 95 us: no gain past 64.
+            const int most = which == 0 && net.layered_max == kLayeredMaxBoards
+                                 ? kLayeredTailBoards
+                                 : net.layered_max;
+            const int rest = which == 0 && layered && !counts && !bits &&
+                                     net.cus > 0 && n > net.cus
+                                 ? n % net.cus
+                                 : 0;
+            if (layered && n <= (counts || bits ? net.layered_max : most)) {
                 e = fused_forward_layered(which, ft, d_planes, args, d_raw,
                                           d_out, n, temperature, ws.tiles,
                                           stream, bits);
-            else
+            } else if (rest > 0 && rest <= most) {
+                const size_t k = n - rest, P = kMaxSide * kMaxSide;
+                e = fused_forward(which, ft, d_planes, args, d_raw, d_out,
+                                  (int)k, temperature, cfg, stream);
+                if (e == hipSuccess)
+                    e = fused_forward_layered(
+                        which, ft, d_planes + k * 32 * P, args,
+                        d_raw ? d_raw + k * P : nullptr,
+                        d_out ? d_out + k * P : nullptr, rest, temperature,
+                        ws.tiles, stream);
+            } else {
                 e = fused_forward(which, ft, d_planes, args, d_raw, d_out, n,
                                   temperature, cfg, stream);
+            }
         }
         if (e == hipSuccess && timer) e = timer->mark(stream);
         if (e != hipSuccess) {

@@ -42,6 +42,35 @@ def test_layered_equals_fused(be, prec, n):
         np.testing.assert_array_equal(out_l, out_f)
 
 
+@pytest.mark.parametrize("n", [65, 96, 97, 256, 257, 352, 353, 513, 600])
+def test_rest_of_a_policy_batch_equals_fused(be, n):
+    """Policy batches of up to 96 boards, and up to 96 boards past whole
+    passes of 256, run in the layered form: the same bits as the persistent
+    kernel's alone, in every row and not past them; also without a raw
+    output."""
+    import torch
+    import leela_amd
+    p = leela_amd.PREC_BF16
+    print(f"case: n={n}", flush=True)
+    planes = torch.from_numpy(make_batch(n, seed0=5000 + n)).cuda()
+    got = {}
+    for lm in (0, 64):
+        be.set_layered_max(lm)
+        raw = torch.full((n + 1, 361), -7.0, device="cuda")
+        out = torch.full((n + 1, 361), -7.0, device="cuda")
+        only = torch.full((n + 1, 361), -7.0, device="cuda")
+        st = torch.cuda.current_stream().cuda_stream
+        be.forward_device(0, p, n, planes.data_ptr(), raw.data_ptr(),
+                          out.data_ptr(), st)
+        be.forward_device(0, p, n, planes.data_ptr(), None, only.data_ptr(),
+                          st)
+        got[lm] = [t.cpu().numpy() for t in (raw, out, only)]
+    be.set_layered_max(64)
+    for a, b in zip(got[0], got[64]):
+        np.testing.assert_array_equal(a, b)
+        assert (b[n] == -7.0).all()
+
+
 def test_layered_queue_bucket_equals_direct(be):
     """16 positions through the queue's 64-board bucket (layered graph,
     device-side count) equal a direct fused forward of the same boards."""
