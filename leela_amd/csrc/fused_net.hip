@@ -700,11 +700,14 @@ hipError_t launch(int which, int wm, const uint8_t *planes,
 // bit.
 constexpr int kLS = 19;
 constexpr int kLMT = 2;  // output m-tiles per workgroup
-// A prefetch distance of the layered convs, in k-steps. Measured at 1 / 16
-// / 64 boards (policy, FP16): 2 steps 97 / 113 / 155 us per forward; 1, 3,
-// 4 and 6 steps 118-122 / 141 / 186 (the value net 93 / 100 / 117 for
-// every distance).
+// A prefetch distance of the layered kernels, in k-steps. Measured at 1 / 16
+// / 64 boards (policy, FP16) with one workgroup a band: 2 steps 97 / 113 /
+// 155 us per forward; 1, 3, 4 and 6 steps 118-122 / 141 / 186 (the value net
+// 93 / 100 / 117 for every distance). With two a band, which leave room for
+// it, 8 steps 72.6 / 84.9 against 2 steps 80.5 / 103 (1 / 16 boards).
 constexpr int kLayeredPF = 2;
+// Most boards whose trunk convs take two workgroups a band.
+constexpr int kSplitPolicy = 25, kSplitValue = 16;
 template <int PS>
 constexpr int lrp() { return (kLS + 2) * PS + row_pad(PS, 2); }
 constexpr int lrp_in() { return (kLS + 4) * kInPS + row_pad(kInPS, 4); }
@@ -722,13 +725,14 @@ typedef const __attribute__((address_space(1))) void gbl_void_t;
 
 // Copies `chunks` KiB from global memory to LDS (both 16-byte aligned) with
 // direct global-to-LDS loads, 16 bytes per lane (no registers, all in
-// flight at once); the waves take chunks round robin. The caller waits
+// flight at once); the WV waves take chunks round robin. The caller waits
 // (vmcnt(0)) and synchronises the workgroup.
+template <int WV = kWN>
 __device__ __forceinline__ void copy_to_lds(const void *src, void *dst,
                                             int chunks, int wave, int lane) {
     const char *g = static_cast<const char *>(src) + lane * 16;
     char *l = static_cast<char *>(dst);
-    for (int c = wave; c < chunks; c += kWN)
+    for (int c = wave; c < chunks; c += WV)
         __builtin_amdgcn_global_load_lds((gbl_void_t *)(g + c * 1024),
                                          (lds_void_t *)(l + c * 1024), 16, 0,
                                          0);
@@ -885,7 +889,7 @@ __device__ __forceinline__ void band_geom(int b, int lane,
 // Stages band b's rows y0 - 1 .. y0 + rows of the board's tile (global
 // rows y0 .. y0 + rows + 1) into LDS: whole KiB chunks directly, the tail
 // through registers.
-template <typename T, int PS>
+template <typename T, int PS, int WV = kWN>
 __device__ __forceinline__ void band_stage(const T *tile, int b, T *s_act,
                                            int tid, int wave, int lane) {
     constexpr int rp = lrp<PS>();
@@ -894,42 +898,48 @@ __device__ __forceinline__ void band_stage(const T *tile, int b, T *s_act,
     const char *src = reinterpret_cast<const char *>(tile + (size_t)y0 * rp);
     const int bytes = rows * rp * (int)sizeof(T);
     const int full = bytes / 1024, tail = bytes % 1024;
-    copy_to_lds(src, s_act, full, wave, lane);
+    copy_to_lds<WV>(src, s_act, full, wave, lane);
     if (tid * 16 < tail)
         reinterpret_cast<uint4 *>(reinterpret_cast<char *>(s_act) +
                                   full * 1024)[tid] =
             reinterpret_cast<const uint4 *>(src + full * 1024)[tid];
 }
 
-// One 3x3 conv CIN -> C of the trunk for one band of one board.
-template <typename T, int PS, int CIN, int C>
-__global__ __launch_bounds__(kWN * 64) void layered_conv(
+// One 3x3 conv CIN -> C of the trunk for one band of one board, by CS
+// workgroups of WV waves that share the output channels. A workgroup streams
+// its channels' weights (295 KB for all 128) through one CU, which is most
+// of its time: while there are CUs to spare, two of them halve it. PF: see
+// DeepConv.
+template <typename T, int PS, int CIN, int C, int CS, int WV, int PF>
+__global__ __launch_bounds__(WV * 64) void layered_conv(
     const T *__restrict__ in_tiles, const void *w,
     const float *__restrict__ bias, T *__restrict__ out_tiles, int n,
     const int *counts) {
     typedef typename Op<T>::v8 v8;
-    constexpr int MT = C / 16, MTW = MT / kWN, TILE = ltile<PS>();
-    static_assert(MT % kWN == 0 && TILE % 512 == 0, "trunk tiling");
+    constexpr int MT = C / 16, MTW = MT / (CS * WV), TILE = ltile<PS>();
+    static_assert(MT % (CS * WV) == 0 && TILE % 512 == 0, "trunk tiling");
     static_assert((lrp<PS>() * (int)sizeof(T)) % 16 == 0 &&
                       (kBandRows + 2) * lrp<PS>() * (int)sizeof(T) % 1024 <=
-                          kWN * 64 * 16,
+                          WV * 64 * 16,
                   "band staging");
-    const int board = blockIdx.x / kBands, b = blockIdx.x % kBands;
+    const int board = blockIdx.x / (kBands * CS);
+    const int b = blockIdx.x / CS % kBands;
     if (board >= layered_boards(n, counts)) return;
     __shared__ __attribute__((aligned(16))) T s_act[(kBandRows + 2) * lrp<PS>()];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    band_stage<T, PS>(in_tiles + (size_t)board * TILE, b, s_act, tid, wave,
-                      lane);
-    DeepConv<T, 3, CIN, MT, MTW, kLayeredPF> dc;
-    dc.prefetch(static_cast<const v8 *>(w), wave * MTW, lane, bias);
+    const int mt0 = ((int)blockIdx.x % CS * WV + wave) * MTW;
+    band_stage<T, PS, WV>(in_tiles + (size_t)board * TILE, b, s_act, tid, wave,
+                          lane);
+    DeepConv<T, 3, CIN, MT, MTW, PF> dc;
+    dc.prefetch(static_cast<const v8 *>(w), mt0, lane, bias);
     int pb[kBandNT], po[kBandNT], pix[kBandNT];
     band_geom<PS>(b, lane, pb, po, pix);
     wait_lds_copies();
     __syncthreads();
     f32x4 acc[MTW][kBandNT];
     dc.template run<PS, kBandNT>(s_act, acc, pb, lrp<PS>(), lane);
-    store_tile<T, MTW, kBandNT>(out_tiles + (size_t)board * TILE, acc,
-                                wave * MTW, po, lane);
+    store_tile<T, MTW, kBandNT>(out_tiles + (size_t)board * TILE, acc, mt0, po,
+                                lane);
 }
 
 // The 1-channel head conv (FP32 accumulation, ELU) of one band of one
@@ -1030,12 +1040,19 @@ hipError_t layered_run(int which, const uint8_t *planes, const FusedArgs &a,
             return hipErrorInvalidValue;
         hipLaunchKernelGGL((layered_stem<T, 144, 96>), dim3(n * 3), blk, 0, s,
                            planes, bits, a.w[0], a.b[0], buf[0], n, cnt);
-        hipLaunchKernelGGL((layered_conv<T, 144, 96, 128>), dim3(n * kBands),
-                           blk, 0, s, buf[0], a.w[1], a.b[1], buf[1], n, cnt);
+        // Two workgroups a band while that is at most one a CU: policy net
+        // 108 -> 73 us at 1 board, 113 -> 85 at 16; at 32 boards 126 -> 128.
+        const int cs = n <= kSplitPolicy ? 2 : 1;
+        const auto first = cs == 2 ? layered_conv<T, 144, 96, 128, 2, kWN, 8>
+                                   : layered_conv<T, 144, 96, 128, 1, kWN, 2>;
+        const auto conv = cs == 2 ? layered_conv<T, 144, 128, 128, 2, kWN, 8>
+                                  : layered_conv<T, 144, 128, 128, 1, kWN, 2>;
+        const dim3 grid(n * kBands * cs);
+        hipLaunchKernelGGL(first, grid, blk, 0, s, buf[0], a.w[1], a.b[1],
+                           buf[1], n, cnt);
         for (int l = 2; l <= 11; l++)
-            hipLaunchKernelGGL((layered_conv<T, 144, 128, 128>),
-                               dim3(n * kBands), blk, 0, s, buf[(l + 1) & 1],
-                               a.w[l], a.b[l], buf[l & 1], n, cnt);
+            hipLaunchKernelGGL(conv, grid, blk, 0, s, buf[(l + 1) & 1], a.w[l],
+                               a.b[l], buf[l & 1], n, cnt);
         hipLaunchKernelGGL((layered_policy_out<T, 144, 128>), dim3(n), blk, 0,
                            s, buf[1], a.w[12], a.b[12], raw, out, n, cnt,
                            temperature);
@@ -1045,10 +1062,15 @@ hipError_t layered_run(int which, const uint8_t *planes, const FusedArgs &a,
         return hipErrorInvalidValue;  // (h0: the value head planes)
     hipLaunchKernelGGL((layered_stem<T, 80, 64>), dim3(n * 2), blk, 0, s,
                        planes, bits, a.w[0], a.b[0], buf[0], n, cnt);
+    // (As above, with two waves each: value net 64.5 -> 60.5 us at 1 board, 68
+    // -> 66 at 16; at 32 boards 70 -> 80.)
+    const int cs = n <= kSplitValue ? 2 : 1;
+    const auto conv = cs == 2 ? layered_conv<T, 80, 64, 64, 2, 2, 4>
+                              : layered_conv<T, 80, 64, 64, 1, kWN, 2>;
     for (int l = 1; l <= 10; l++)
-        hipLaunchKernelGGL((layered_conv<T, 80, 64, 64>), dim3(n * kBands),
-                           blk, 0, s, buf[(l + 1) & 1], a.w[l], a.b[l],
-                           buf[l & 1], n, cnt);
+        hipLaunchKernelGGL(conv, dim3(n * kBands * cs), dim3(kWN * 64 / cs), 0,
+                           s, buf[(l + 1) & 1], a.w[l], a.b[l], buf[l & 1], n,
+                           cnt);
     hipLaunchKernelGGL((layered_head<T, 80, 64>), dim3(n * kBands), blk, 0, s,
                        buf[0], a.w[11], a.b[11], a.h0, n, cnt);
     hipError_t e = hipGetLastError();

@@ -42,6 +42,24 @@ def test_layered_equals_fused(be, prec, n):
         np.testing.assert_array_equal(out_l, out_f)
 
 
+@pytest.mark.parametrize("n", [2, 16, 17, 25, 26])
+def test_layered_equals_fused_where_bands_split(be, n):
+    """Small batches run a band's channels in two workgroups (policy up to 25
+    boards, value up to 16): the same bits as the persistent kernels."""
+    import leela_amd
+    print(f"case: n={n}", flush=True)
+    for prec in (leela_amd.PREC_BF16, leela_amd.PREC_FP16):
+        for net in (leela_amd.NET_POLICY, leela_amd.NET_VALUE):
+            planes = make_batch(n, seed0=7000 + n, net=net)
+            be.set_layered_max(64)
+            got = be.forward(net, prec, planes)
+            be.set_layered_max(0)
+            want = be.forward(net, prec, planes)
+            be.set_layered_max(64)
+            for a, b in zip(got, want):
+                np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("n", [65, 96, 97, 256, 257, 352, 353, 513, 600])
 def test_rest_of_a_policy_batch_equals_fused(be, n):
     """Policy batches of up to 96 boards, and up to 96 boards past whole
