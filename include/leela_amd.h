@@ -38,7 +38,8 @@ extern "C" {
 #define LZ_NET_POLICY 0
 #define LZ_NET_VALUE 1
 
-#define LZ_PREC_FP32 0 /* plain form: FP32 everywhere, FP32 MFMA */
+#define LZ_PREC_FP32 0 /* plain form: FP32 everywhere (its products as three-
+                          part BF16 ones on MFMA, exact to 2^-25) */
 #define LZ_PREC_BF16 1 /* BF16 trunk on MFMA, FP32 accumulate/epilogue */
 #define LZ_PREC_FP8 2  /* FP8 e4m3 operands after the 5x5 stem (FP16):
                           per-output-channel weight scales, per-board
@@ -345,7 +346,7 @@ int lz_encode_batch(const lz_position *const *pos, int n, int net,
                     int symmetry, int threads, uint8_t *planes);
 
 /* ---- Device feature encoder -------------------------------------------
- * The same planes computed on the GPU, one wavefront per board, written
+ * The same planes computed on the GPU, one to four wavefronts per board, written
  * straight into device memory where the nets read them: the per-leaf
  * gather_features_policy / gather_features_value calls (Network.cpp:557,
  * 597, 633; encoders at :883-1201) moved off the host. The host side only
@@ -560,13 +561,13 @@ int lz_playout_scores(const lz_position *pos, int policy, int n,
                       uint32_t seed, float *scores);
 
 /* lz_playout_winrates_device with the chosen playout policy. With
- * LZ_PLAYOUT_PATTERN each playout runs on one GPU thread, the same source
+ * LZ_PLAYOUT_PATTERN each playout runs on one wavefront, the same source
  * as the host's (its win rates equal lz_playout_winrate_policy's for the
  * same position and seed); a position whose candidate list outgrows the
  * device's 2,048 entries (none of millions of generator positions' move
  * generations needs more than ~300) gets NaN instead of a win rate. The
- * first pattern call uploads the tables and allocates ~4.5 GB of playout
- * states (one per thread of a persistent grid of 196,608 threads), held
+ * first pattern call uploads the tables and allocates 81 MB of long
+ * candidate lists (one per wavefront of a persistent grid of 5,120), held
  * until lz_encoder_destroy. Pattern calls on one encoder are ordered by
  * the library, whatever their streams. */
 int lz_playout_winrates_device_policy(lz_encoder *enc,
@@ -650,7 +651,8 @@ int lz_surrogate_train_step_device(lz_surrogate *s, int n,
  * checks. kind 0: the BF16 output map [n][361][64] of conv `layer` (0..12,
  * after ELU); kind 1: the BF16 gradient map at that conv's pre-activation,
  * available once lz_surrogate_keep_maps(s, 1) has been set (it keeps all
- * 13 maps instead of 3 rotating ones). Values are raw BF16 bit patterns.
+ * 13 maps of max_batch boards instead of at most 1024). Values are raw
+ * BF16 bit patterns.
  * lz_surrogate_read_head copies the head's saved s [n][361], f [n][64] and
  * t [n] (any pointer may be NULL). */
 int lz_surrogate_keep_maps(lz_surrogate *s, int on);

@@ -216,7 +216,7 @@ def _as_array(positions):
 
 class DeviceEncoder:
     """The feature encoder on the GPU (lz_encode_device): planes of a batch
-    of Position objects written into device memory, one wavefront per
+    of Position objects written into device memory, one to four wavefronts per
     board. Sides may differ within a batch (planes packed board after
     board)."""
 
