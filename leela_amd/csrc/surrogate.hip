@@ -12,11 +12,14 @@
 //   FP32 epilogue adds bias and residual and applies ELU.
 //   Bound: MFMA and its operand reads from n = 512 up (333 MFLOP a board),
 //   with the maps' stores (0.6 MB a board) beside them; one conv's latency,
-//   13 times, below one board per CU. At n = 4096: 1.32 ms (1.03 PFLOP/s;
-//   1.09 ms with the stores taken out), against 3.37 ms for one launch per
-//   conv with its input staged from HBM each time. Residuals read back from
-//   HBM instead of kept in registers cost 0.7 ms of the 4096, stores of 8
-//   bytes straight from the accumulators 0.4 ms.
+//   13 times, below one board per CU. At n = 4096: 1.61 ms (0.84 PFLOP/s),
+//   against 3.37 ms for one launch per conv with its input staged from HBM
+//   each time, with the same outputs to the bit: sums in the same order, the
+//   library's expf. (The hardware base-2 exponential of a rounded product in
+//   its place takes 0.28 ms less, but its absolute error is 6.9e-8 at most
+//   against 4.5e-8.) Residuals read back from HBM instead of kept in
+//   registers cost 0.7 ms of the 4096, stores of 8 bytes straight from the
+//   accumulators 0.4 ms.
 //
 // Backward-data — sg_bwd
 //   The same for the backward pass: one launch, a board's gradient map in
@@ -24,10 +27,10 @@
 //   W'[c][o][tap] = W[o][c][8 - tap] (taps flipped), packed by sg_pack; the
 //   epilogue adds the skip's gradient (kept in registers), multiplies by
 //   ELU's derivative taken from the stored forward activation, and the map
-//   goes to HBM for the weight gradients. n = 512: 228 us against 440 for
-//   one launch per conv and 306 for the head's; 98 us at n = 61. The mask
-//   map's trip through registers after each conv is what it takes over the
-//   forward pass's 170.
+//   goes to HBM for the weight gradients. n = 512: 242 us against 440 for
+//   one launch per conv and 306 for the head's (the forward pass 215); 97 us
+//   at n = 61. Besides the MFMAs it takes the mask map's trip through
+//   registers after each conv.
 //
 // Weight gradients — sg_wgrad
 //   dW[o][c][tap] = sum over boards and pixels of e[p][o] x[p + tap][c]: a
@@ -40,7 +43,7 @@
 //   taps x 64 output channels (144 accumulators) over half the pixels.
 //   sg_reduce sums the partials in a fixed order (deterministic) into OIHW.
 //   Bound at n = 512: 0.7 GB of maps read (134 us at this card's copy rate)
-//   and 173 GFLOP; 208 us, of which the copies alone take 140 and the MFMAs
+//   and 173 GFLOP; 213-229 us, of which the copies alone take 140 and the MFMAs
 //   alone 137 (two buffers do not hide all of the one behind the other; a
 //   k-step's copies issued between its MFMAs instead of ahead of them
 //   measured 217). Nine transposed copies of each map, one per tap, took
@@ -65,9 +68,9 @@ constexpr int kThreads = 256;
 constexpr int kMaxChunks = 19;
 constexpr int kPart = 9 * kCh * kCh;  // floats of a weight-gradient partial
 // Batches of at most this many boards (one per CU) use eight waves a board:
-// 95 us up to n = 200 and 102 at 256, against 122-124 with four; from 257 on
-// a CU holds two boards and four waves each are faster (152 against 173 us
-// at 257, 332 against 354 at 1024).
+// 116 us at n = 1 and 121 at 256, against 155-158 with four; from 257 on
+// a CU holds two boards and four waves each are faster (193 against 213 us
+// at 257, 405 against 429 at 1024).
 constexpr int kWideBoards = 256;
 
 __device__ inline f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -151,28 +154,32 @@ __device__ __forceinline__ void sg_geom(int wn, int lane, int (&pb)[kNT],
     }
 }
 
-// Epilogue of a forward conv (bias in the accumulators): + residual, ELU,
-// BF16 into the tile. acc's lane holds four consecutive channels of one
-// pixel per fragment. keep: the lane's outputs of the last even conv, which
-// are the residual of an even conv (kRes) and are replaced by its outputs
-// (kKeep).
+// Epilogue of a forward conv: + bias, + residual, ELU, BF16 into the tile.
+// acc's lane holds four consecutive channels of one pixel per fragment.
+// bias: the conv's 64, in LDS. keep: the lane's outputs of the last even
+// conv, which are the residual of an even conv (kRes) and are replaced by its
+// outputs (kKeep). (The sums in this order and the library's expf: the
+// outputs are to the bit those of one launch per conv.)
 template <bool kRes, bool kKeep, int MTW>
 __device__ __forceinline__ void sg_store_fwd(__bf16 *tile,
                                              const f32x4 (&acc)[MTW][kNT],
                                              bf16x4 (&keep)[MTW][kNT],
-                                             int mt0, const int (&pb)[kNT],
+                                             const float *bias, int mt0,
+                                             const int (&pb)[kNT],
                                              const int (&pix)[kNT], int lane) {
     const int g4 = (lane >> 4) * 4;
 #pragma unroll
     for (int m = 0; m < MTW; m++) {
         const int o = (mt0 + m) * 16 + g4;
+        const f32x4 bo = *(const f32x4 *)(bias + o);
 #pragma unroll
         for (int t = 0; t < kNT; t++) {
             bf16x4 v;
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                v[r] = (__bf16)elu_operand(
-                    kRes ? acc[m][t][r] + (float)keep[m][t][r] : acc[m][t][r]);
+            for (int r = 0; r < 4; r++) {
+                const float d = acc[m][t][r] + bo[r];
+                v[r] = (__bf16)elu(kRes ? d + (float)keep[m][t][r] : d);
+            }
             if (kKeep) keep[m][t] = v;
             if (pix[t] >= 0)
                 *(bf16x4 *)(tile + pb[t] + kRP + kPS + o) = v;
@@ -214,11 +221,15 @@ __global__ __launch_bounds__(kWM * kThreads, 2) void sg_fwd(
     __shared__ __attribute__((aligned(16))) __bf16 tile[kTile];
     __shared__ float s[P];
     __shared__ float f[kHid];
+    __shared__ __attribute__((aligned(16))) float s_bias[kNConv * kCh];
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int mt0 = (w / kWN) * MTW;
     const bf16x8 zero8 = {};
     __bf16 *maps = (__bf16 *)act + (size_t)b * P * kCh;
 
+#pragma unroll
+    for (int l = 0; l < kNConv; l++)
+        if (tid < kCh) s_bias[l * kCh + tid] = a.b[l][tid];
     // The planes with a zero halo: a thread takes 8 planes of a point.
     const uint8_t *pl = planes + (size_t)b * 32 * P;
     for (int i = tid; i < HP * 4; i += T) {
@@ -243,12 +254,13 @@ __global__ __launch_bounds__(kWM * kThreads, 2) void sg_fwd(
         for (int t = 0; t < kNT; t++)
             pbi[t] = pb[t] / kRP * kInRP + pb[t] % kRP / kPS * kInPS;
         conv_tile<__bf16, 3, 32, MT, MTW, kInPS>(
-            tile, (const bf16x8 *)a.w[0], acc, pbi, kInRP, mt0, lane, a.b[0]);
+            tile, (const bf16x8 *)a.w[0], acc, pbi, kInRP, mt0, lane);
         __syncthreads();
         for (int i = tid * 8; i < kTile; i += T * 8)
             *(bf16x8 *)(tile + i) = zero8;
         __syncthreads();
-        sg_store_fwd<false, true, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        sg_store_fwd<false, true, MTW>(tile, acc, keep, s_bias, mt0, pb, pix,
+                                       lane);
         __syncthreads();
     }
     // The map of a conv's input goes out between its MFMAs and its epilogue:
@@ -257,17 +269,18 @@ __global__ __launch_bounds__(kWM * kThreads, 2) void sg_fwd(
     for (int l = 1; l < kNConv; l += 2) {
         f32x4 acc[MTW][kNT];
         conv_tile<__bf16, 3, kCh, MT, MTW, kPS>(
-            tile, (const bf16x8 *)a.w[l], acc, pb, kRP, mt0, lane, a.b[l]);
+            tile, (const bf16x8 *)a.w[l], acc, pb, kRP, mt0, lane);
         sg_copy_out<T, kStream>(tile, maps + (l - 1) * map_elems, tid);
         __syncthreads();
-        sg_store_fwd<false, false, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        sg_store_fwd<false, false, MTW>(tile, acc, keep, s_bias + l * kCh, mt0,
+                                        pb, pix, lane);
         __syncthreads();
         conv_tile<__bf16, 3, kCh, MT, MTW, kPS>(
-            tile, (const bf16x8 *)a.w[l + 1], acc, pb, kRP, mt0, lane,
-            a.b[l + 1]);
+            tile, (const bf16x8 *)a.w[l + 1], acc, pb, kRP, mt0, lane);
         sg_copy_out<T, kStream>(tile, maps + l * map_elems, tid);
         __syncthreads();
-        sg_store_fwd<true, true, MTW>(tile, acc, keep, mt0, pb, pix, lane);
+        sg_store_fwd<true, true, MTW>(tile, acc, keep, s_bias + (l + 1) * kCh,
+                                      mt0, pb, pix, lane);
         __syncthreads();
     }
     sg_copy_out<T, kStream>(tile, maps + (kNConv - 1) * map_elems, tid);

@@ -175,6 +175,48 @@ def test_gradient_of_a_batch_is_the_mean_of_its_halves(k):
                                    err_msg=name)
 
 
+@pytest.mark.parametrize("n", [1, 257])
+def test_activation_is_the_float32_elu(n):
+    """With zero weights a conv's pre-activation is its bias, so its map is
+    ELU(bias) = expf(bias) - 1 in FP32, rounded once to BF16: to the bit
+    what torch forms from its float32 exponential. The biases are values
+    whose BF16 result is another one if the exponential is formed as 2 to the
+    rounded product with log2 e, which is off by up to an ulp more."""
+    import torch
+    print(f"surrogate ELU: {n} boards", flush=True)
+
+    def result(e, v):
+        return torch.where(v > 0, v, e - 1).bfloat16().view(torch.int16)
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    v = -torch.exp2(torch.rand(1 << 24, generator=g, device="cuda") * 16 - 12)
+    want = result(torch.exp(v), v)
+    at = (want != result(torch.exp2(v * 1.4426950408889634), v)).nonzero()[:, 0]
+    assert len(at) > 0
+    plain = torch.tensor([1.5, 0.0, -0.5, -3.0, -20.0, -200.0], device="cuda")
+    v = torch.cat([v[at], plain])
+    want = result(torch.exp(v), v).cpu().numpy().view(np.uint16)
+    v = v.cpu().numpy()
+    planes = np.zeros((n, 32, 361), np.uint8)
+    free = [0, *range(1, orc.NCONV, 2)]  # convs without a residual
+    offs = {name: off for name, _, off in orc.layout()}
+    s = Surrogate(0, max_batch=n, seed=3)
+    try:
+        for k in range(0, min(len(v), 2048), 64 * len(free)):
+            idx = (np.arange(64 * len(free)) + k) % len(v)
+            flat = np.zeros(orc.num_params(), np.float32)
+            for l, i in zip(free, idx.reshape(len(free), 64)):
+                flat[offs[f"b{l}"]:offs[f"b{l}"] + 64] = v[i]
+            s.set_params(flat)
+            s.predict(planes)
+            for l, i in zip(free, idx.reshape(len(free), 64)):
+                got = s.read_map(0, l, n)
+                np.testing.assert_array_equal(
+                    got, np.broadcast_to(want[i], got.shape), err_msg=str(l))
+    finally:
+        s.close()
+
+
 def _bf(u16):
     """BF16 bit patterns -> float64."""
     return (u16.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
