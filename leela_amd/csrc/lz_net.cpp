@@ -370,10 +370,38 @@ void free_net(Net &net) {
     }
 }
 
+namespace {
+
+// The buffers that growth replaces.
+void free_activations(Workspace &ws) {
+    dfree(ws.planes);
+    dfree(ws.act[0]);
+    dfree(ws.act[1]);
+    dfree(ws.raw);
+    dfree(ws.out);
+    ws.planes = nullptr;
+    ws.act[0] = ws.act[1] = ws.raw = ws.out = nullptr;
+    ws.cap = 0;
+}
+
+hipError_t grow_h0(Workspace &ws, int n) {
+    if (n <= ws.h0_cap) return hipSuccess;
+    const int cap = ws.h0_cap > n / 2 ? 2 * ws.h0_cap : n;
+    float *p = nullptr;
+    const hipError_t e = dalloc(&p, (size_t)cap * kMaxSide * kMaxSide);
+    if (e != hipSuccess) return e;
+    if (ws.h0) ws.old_h0[ws.n_old_h0++] = ws.h0;
+    ws.h0 = p;
+    ws.h0_cap = cap;
+    return hipSuccess;
+}
+
+}  // namespace
+
 int ensure_workspace(Workspace &ws, const Net nets[2], int n,
                      std::string *msg) {
     if (n <= ws.cap) return LZ_OK;
-    free_workspace(ws);
+    free_activations(ws);
     int ch = 32;
     int cin0 = 0;
     for (int k = 0; k < 2; k++) {
@@ -388,9 +416,9 @@ int ensure_workspace(Workspace &ws, const Net nets[2], int n,
     if (e == hipSuccess) e = dalloc(&ws.act[1], (size_t)n * ch * P);
     if (e == hipSuccess) e = dalloc(&ws.raw, (size_t)n * P);
     if (e == hipSuccess) e = dalloc(&ws.out, (size_t)n * P);
-    if (e == hipSuccess) e = dalloc(&ws.h0, (size_t)n * P);
+    if (e == hipSuccess) e = grow_h0(ws, n);
     if (e != hipSuccess) {
-        free_workspace(ws);
+        free_activations(ws);
         *msg = std::string("workspace allocation: ") + hipGetErrorString(e);
         return LZ_ERR_NOMEM;
     }
@@ -413,12 +441,9 @@ int ensure_tiles(Workspace &ws, std::string *msg) {
 }
 
 void free_workspace(Workspace &ws) {
-    dfree(ws.planes);
-    dfree(ws.act[0]);
-    dfree(ws.act[1]);
-    dfree(ws.raw);
-    dfree(ws.out);
+    free_activations(ws);
     dfree(ws.h0);
+    for (int i = 0; i < ws.n_old_h0; i++) dfree(ws.old_h0[i]);
     if (ws.tiles) (void)hipFree(ws.tiles);
     ws = Workspace();
 }

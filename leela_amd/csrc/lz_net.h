@@ -73,13 +73,21 @@ struct Net {
 int tune_bucket(int n);
 FusedLaunch fused_launch_for(const Net &net, int which, int nslots);
 
+// What the 16-bit and FP8 forms use (h0, tiles) stays allocated when the
+// workspace grows: a captured forward may hold its address and be replayed
+// after a larger batch. Each h0 has at least twice the rows of the one
+// before, so that the kept ones take less than the last. The rest belongs to
+// the FP32 form and the host entry points and is replaced.
 struct Workspace {
     int cap = 0;             // positions the buffers hold
     uint8_t *planes = nullptr;
     float *act[2] = {nullptr, nullptr};
     float *raw = nullptr;
     float *out = nullptr;
-    float *h0 = nullptr;     // value head plane [cap][361]
+    float *h0 = nullptr;     // value head plane [h0_cap][361]
+    int h0_cap = 0;
+    float *old_h0[31] = {};  // the smaller ones before it
+    int n_old_h0 = 0;
     void *tiles = nullptr;   // layered form's activation tiles (zeroed)
 };
 

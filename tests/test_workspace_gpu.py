@@ -59,3 +59,73 @@ def test_two_streams_two_workspaces(be, na, nb):
         finally:
             be.free_workspace(w1)
             be.free_workspace(w2)
+
+
+@pytest.mark.parametrize("own", [False, True])
+def test_captured_forwards_outlive_growth(weights_a, own):
+    """16-bit forwards captured before the workspace grows (the policy's
+    layered tiles: small batches, batches of 65..96 and the rest past a pass
+    of 256; the value net's head planes) give the same results when they are
+    replayed after it has grown, several times, with eager work between the
+    replays."""
+    import torch
+    import leela_amd
+    p = leela_amd.PREC_FP16
+    be = leela_amd.Backend(0)
+    for net, w in enumerate(weights_a):
+        be.load_net(net, w)
+    be.finalize()
+    ws = be.workspace(8) if own else None
+
+    def forward(net, n, d, raw, out, stream):
+        args = (net, p, n, d.data_ptr(), raw.data_ptr(), out.data_ptr(),
+                stream.cuda_stream)
+        if own:
+            be.forward_device_ws(ws, *args)
+        else:
+            be.forward_device(*args)
+
+    def case(net, n):
+        print(f"case: own={own} net={net} n={n}", flush=True)
+        d = torch.from_numpy(make_batch(n, seed0=300 + n, net=net)).cuda()
+        width = 361 if net == leela_amd.NET_POLICY else 1
+        return (net, n, d, torch.empty((n, width), device="cuda"),
+                torch.empty((n, width), device="cuda"))
+
+    st = torch.cuda.Stream()
+    cases = [case(0, 16), case(0, 80), case(0, 300), case(1, 300)]
+    torch.cuda.synchronize()
+    for c in cases:
+        forward(*c, st)
+    st.synchronize()
+    want = [(c[3].cpu().numpy(), c[4].cpu().numpy()) for c in cases]
+    graphs = []
+    for c in cases:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            forward(*c, torch.cuda.current_stream())
+        graphs.append(g)
+    held = []
+    for n in (420, 1500):
+        big = [case(0, n), case(1, n)]
+        torch.cuda.synchronize()
+        for _ in range(2):
+            for c in big:
+                forward(*c, st)
+            # Takes what the growth has given back.
+            held += [torch.full((1 << 22,), -1, dtype=torch.int32,
+                                device="cuda") for _ in range(8)]
+            for c, g, w in zip(cases, graphs, want):
+                c[3].fill_(-7.0)
+                c[4].fill_(-7.0)
+                torch.cuda.synchronize()
+                with torch.cuda.stream(st):
+                    g.replay()
+                st.synchronize()
+                np.testing.assert_array_equal(c[3].cpu().numpy(), w[0])
+                np.testing.assert_array_equal(c[4].cpu().numpy(), w[1])
+        assert all(bool((t == -1).all()) for t in held)
+    del graphs
+    if own:
+        be.free_workspace(ws)
+    be.close()
