@@ -127,7 +127,8 @@ int lz_forward(lz_ctx *ctx, int net, int precision, int n,
  * (a hipStream_t; NULL is the HIP default stream, as in every HIP call);
  * returns after enqueueing. Buffers must stay valid until the stream
  * reaches the work. Device-buffer calls on one context share its
- * workspace: calls on different streams must be ordered by the caller.
+ * workspace: calls on different streams must be ordered by the caller
+ * (lz_forward has a workspace of its own and needs no ordering).
  * The workspace grows to the largest batch it is given. A forward captured
  * in a HIP graph (of a batch that an earlier call has made room for) stays
  * valid through later growth in the 16-bit and FP8 forms; in LZ_PREC_FP32 a

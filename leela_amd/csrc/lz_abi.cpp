@@ -36,7 +36,7 @@ void set_init_err(const std::string &s) {
 
 namespace lz {
 
-int forward_locked(lz_ctx *ctx, int net, int precision, int n,
+int forward_locked(lz_ctx *ctx, Workspace &ws, int net, int precision, int n,
                    const uint8_t *d_planes, float *d_raw, float *d_out,
                    hipStream_t stream, LaunchTimer *timer) {
     if (!ctx->finalized)
@@ -49,10 +49,10 @@ int forward_locked(lz_ctx *ctx, int net, int precision, int n,
     if (n == 0) return LZ_OK;
     if (!d_planes) return ctx->fail(LZ_ERR_ARG, "planes is NULL");
     std::string msg;
-    int rc = ensure_workspace(ctx->ws, ctx->net, n, &msg);
+    int rc = ensure_workspace(ws, ctx->net, n, &msg);
     if (rc != LZ_OK) return ctx->fail(rc, "%s", msg.c_str());
     rc = run_net(ctx->net[net], net, precision, n, d_planes, d_raw, d_out,
-                 ctx->temperature, ctx->ws, stream, &msg, timer);
+                 ctx->temperature, ws, stream, &msg, timer);
     if (rc != LZ_OK) return ctx->fail(rc, "%s", msg.c_str());
     return LZ_OK;
 }
@@ -334,8 +334,8 @@ int lz_forward_timed(lz_ctx *ctx, int net, int precision, int n,
     (void)hipSetDevice(ctx->device);
     hipStream_t s = static_cast<hipStream_t>(stream);  // NULL: default stream
     lz::LaunchTimer timer;
-    int rc = forward_locked(ctx, net, precision, n, d_planes, d_raw, d_out, s,
-                            &timer);
+    int rc = forward_locked(ctx, ctx->ws, net, precision, n, d_planes, d_raw,
+                            d_out, s, &timer);
     if (rc != LZ_OK) return rc;
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess)
@@ -359,7 +359,8 @@ int lz_forward_device(lz_ctx *ctx, int net, int precision, int n,
     std::lock_guard<std::mutex> g(ctx->mu);
     (void)hipSetDevice(ctx->device);
     hipStream_t s = static_cast<hipStream_t>(stream);  // NULL: default stream
-    return forward_locked(ctx, net, precision, n, d_planes, d_raw, d_out, s);
+    return forward_locked(ctx, ctx->ws, net, precision, n, d_planes, d_raw,
+                          d_out, s);
 }
 
 }  // extern "C"
@@ -441,9 +442,9 @@ int lz_forward(lz_ctx *ctx, int net, int precision, int n,
         return ctx->fail(LZ_ERR_STATE, "forward before lz_finalize");
     (void)hipSetDevice(ctx->device);
     std::string msg;
-    int rc = lz::ensure_workspace(ctx->ws, ctx->net, n, &msg);
+    lz::Workspace &ws = ctx->host_ws;
+    int rc = lz::ensure_workspace(ws, ctx->net, n, &msg);
     if (rc != LZ_OK) return ctx->fail(rc, "%s", msg.c_str());
-    lz::Workspace &ws = ctx->ws;
     const lz::Net &N = ctx->net[net < 0 || net > 1 ? 0 : net];
     const int cin0 = N.layers.empty() ? 0 : N.layers[0].cin;
     const size_t in_bytes = (size_t)n * cin0 * N.side * N.side;
@@ -451,7 +452,7 @@ int lz_forward(lz_ctx *ctx, int net, int precision, int n,
                                   hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess)
         return ctx->fail(LZ_ERR_HIP, "H2D planes: %s", hipGetErrorString(e));
-    rc = forward_locked(ctx, net, precision, n, ws.planes, ws.raw, ws.out,
+    rc = forward_locked(ctx, ws, net, precision, n, ws.planes, ws.raw, ws.out,
                         ctx->stream);
     if (rc != LZ_OK) return rc;
     const size_t per = net == LZ_NET_POLICY ? (size_t)N.side * N.side : 1;
@@ -492,6 +493,7 @@ void lz_destroy(lz_ctx *ctx) {
     lz::free_net(ctx->net[0]);
     lz::free_net(ctx->net[1]);
     lz::free_workspace(ctx->ws);
+    lz::free_workspace(ctx->host_ws);
     lz::free_ragged_layout(ctx->ragged);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;

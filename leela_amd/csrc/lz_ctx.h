@@ -22,7 +22,10 @@ struct lz_ctx {
     std::string err;
     std::mutex mu;  // guards the nets, workspace and err
     lz::Net net[2];
-    lz::Workspace ws;
+    lz::Workspace ws;       // device-buffer calls'
+    // lz_forward's own: it runs on `stream`, which a caller of device-buffer
+    // calls on other streams cannot order against.
+    lz::Workspace host_ws;
     lz::RaggedLayout ragged;  // layout of the last ragged batch
     float temperature = 0.75f;
     bool finalized = false;
@@ -40,8 +43,9 @@ struct lz_ctx {
 };
 
 namespace lz {
-// Forward of `net` on device buffers with ctx->mu held (lz_abi.cpp).
-int forward_locked(lz_ctx *ctx, int net, int precision, int n,
+// Forward of `net` on device buffers, with the workspace ws of ctx and with
+// ctx->mu held (lz_abi.cpp).
+int forward_locked(lz_ctx *ctx, Workspace &ws, int net, int precision, int n,
                    const uint8_t *d_planes, float *d_raw, float *d_out,
                    hipStream_t stream, LaunchTimer *timer = nullptr);
 // Stops and frees the leaf queue of ctx, if any (lz_queue.cpp).

@@ -129,3 +129,47 @@ def test_captured_forwards_outlive_growth(weights_a, own):
     if own:
         be.free_workspace(ws)
     be.close()
+
+
+def test_host_forward_beside_device_forwards(weights_a):
+    """lz_forward runs on the context's own stream, which a caller cannot
+    order against: with device-buffer batches of the same context on the way
+    on another stream (layered tiles and head planes in use on both), every
+    result is that of the calls made alone."""
+    import torch
+    import leela_amd
+    p = leela_amd.PREC_FP16
+    be = leela_amd.Backend(0)
+    for net, w in enumerate(weights_a):
+        be.load_net(net, w)
+    be.finalize()
+    try:
+        for net, width, na, nb in ((0, 361, 331, 96), (0, 361, 40, 20),
+                                   (1, 1, 600, 50)):
+            print(f"case: net={net} device n={na} host n={nb}", flush=True)
+            pa = make_batch(na, seed0=11, net=net)
+            pb = make_batch(nb, seed0=77, net=net)
+            want_b = be.forward(net, p, pb)
+            da = torch.from_numpy(pa).cuda()
+            outs = [torch.empty((2, na, width), device="cuda")
+                    for _ in range(21)]
+            st = torch.cuda.Stream()
+            torch.cuda.synchronize()
+
+            def device(o):
+                be.forward_device(net, p, na, da.data_ptr(), o[0].data_ptr(),
+                                  o[1].data_ptr(), st.cuda_stream)
+
+            device(outs[20])
+            st.synchronize()
+            for k in range(5):
+                for o in outs[4 * k:4 * k + 4]:
+                    device(o)
+                got = be.forward(net, p, pb)
+                for a, b in zip(got, want_b):
+                    np.testing.assert_array_equal(a, b)
+            st.synchronize()
+            for o in outs[:20]:
+                assert torch.equal(o, outs[20])
+    finally:
+        be.close()
