@@ -22,7 +22,9 @@ constexpr int kPos = 32 * 361;
 const char *kNetName[2] = {"policy", "value"};
 
 // Milliseconds of one forward (median of 5 after 2 warm-ups); a ragged
-// batch when `ragged` is given.
+// batch when `ragged` is given. Without layered tiles, so that the persistent
+// kernels run in batches of any size: it is their shape that is timed, for
+// every batch of the bucket, ragged ones and queue graphs among them.
 int time_forward(lz_ctx *ctx, int net, int precision, int n,
                  const uint8_t *d_planes, float *d_raw, float *d_out,
                  float *ms_out, std::string *msg,
@@ -33,13 +35,15 @@ int time_forward(lz_ctx *ctx, int net, int precision, int n,
         return LZ_ERR_HIP;
     }
     std::vector<float> t;
+    lz::Workspace ws = ctx->ws;
+    ws.tiles = nullptr;
     int rc = LZ_OK;
     for (int rep = 0; rep < 7 && rc == LZ_OK; rep++) {
         hipError_t e = hipEventRecord(a, ctx->stream);
         if (e == hipSuccess)
             rc = lz::run_net(ctx->net[net], net, precision, n, d_planes, d_raw,
-                             d_out, ctx->temperature, ctx->ws, ctx->stream,
-                             msg, nullptr, ragged);
+                             d_out, ctx->temperature, ws, ctx->stream, msg,
+                             nullptr, ragged);
         if (rc == LZ_OK && e == hipSuccess) e = hipEventRecord(b, ctx->stream);
         if (rc == LZ_OK && e == hipSuccess) e = hipEventSynchronize(b);
         float ms = 0.0f;

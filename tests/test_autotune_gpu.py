@@ -43,3 +43,31 @@ def test_autotune_choice_and_results(weights_a, tmp_path):
         assert open(path).read() == text
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("n", [16, 80, 300])
+def test_autotune_times_the_persistent_kernels(weights_a, n):
+    """Batches that forwards run in the layered form, wholly (16, 80) or in
+    part (300), are tuned on the persistent kernels all the same: the choice
+    serves the other batches of the bucket. Best candidates with the layered
+    form allowed and forbidden then take the same time (the policy net's
+    layered form takes 0.4 of it at 16 boards, 0.8 at 80)."""
+    import leela_amd
+    be = leela_amd.Backend(0)
+    pol, val = weights_a
+    be.load_net(leela_amd.NET_POLICY, pol)
+    be.load_net(leela_amd.NET_VALUE, val)
+    be.finalize()
+    ms = {}
+    try:
+        for limit in (64, 0):
+            be.set_layered_max(limit)
+            be.autotune(leela_amd.PREC_BF16, n)  # (clocks up)
+            for ln in be.autotune(leela_amd.PREC_BF16, n).splitlines():
+                if "chosen" in ln:
+                    ms[ln.split()[0], limit] = float(ln.split()[-2])
+    finally:
+        be.close()
+    print(ms, flush=True)
+    for net in ("policy", "value"):
+        assert ms[net, 64] > 0.9 * ms[net, 0]
