@@ -225,7 +225,8 @@ class Backend:
 
     def set_layered_max(self, max_boards: int):
         """lz_set_layered_max: batches of at most max_boards 19x19
-        positions run the layered 16-bit form (0: never)."""
+        positions run the layered 16-bit form (0: never), and no others;
+        without a call 64, and policy batches up to 96 and rests."""
         self._check(self._L.lz_set_layered_max(self._ctx, max_boards),
                     "lz_set_layered_max")
 

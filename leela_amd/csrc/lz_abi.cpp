@@ -242,7 +242,10 @@ int lz_set_layered_max(lz_ctx *ctx, int max_boards) {
         return ctx->fail(LZ_ERR_ARG, "layered batch limit %d outside 0..%d",
                          max_boards, lz::kLayeredMaxBoards);
     std::lock_guard<std::mutex> g(ctx->mu);
-    for (auto &n : ctx->net) n.layered_max = max_boards;
+    for (auto &n : ctx->net) {
+        n.layered_max = max_boards;
+        n.layered_tail = 0;
+    }
     return LZ_OK;
 }
 

@@ -561,7 +561,7 @@ int run_net(const Net &net, int which, int precision, int n,
         if (e == hipSuccess) {
             // (The layered stem copies planes 16 bytes at a time.)
             const bool layered =
-                !ragged && ws.tiles && net.layered_max > 0 &&
+                !ragged && ws.tiles &&
                 reinterpret_cast<uintptr_t>(d_planes) % 16 == 0;
             // The persistent policy kernel takes a pass of the chip (a board
             // per CU) as long for a few boards as for all: 205 us up to 200
@@ -571,18 +571,17 @@ int run_net(const Net &net, int which, int precision, int n,
             // bits): 257 boards 426 -> 335 us, 331 435 -> 399, 352 439 ->
             // 417, 600 680 -> 653. The value net's passes are of 512 boards
             // and 95 us: no gain past 64.
-            const int most = which == 0 && net.layered_max == kLayeredMaxBoards
-                                 ? kLayeredTailBoards
-                                 : net.layered_max;
-            const int rest = which == 0 && layered && !counts && !bits &&
-                                     net.cus > 0 && n > net.cus
+            const int tail = which == 0 && !counts && !bits
+                                 ? net.layered_tail
+                                 : 0;
+            const int rest = layered && net.cus > 0 && n > net.cus
                                  ? n % net.cus
                                  : 0;
-            if (layered && n <= (counts || bits ? net.layered_max : most)) {
+            if (layered && n <= std::max(net.layered_max, tail)) {
                 e = fused_forward_layered(which, ft, d_planes, args, d_raw,
                                           d_out, n, temperature, ws.tiles,
                                           stream, bits);
-            } else if (rest > 0 && rest <= most) {
+            } else if (rest > 0 && rest <= tail) {
                 const size_t k = n - rest, P = kMaxSide * kMaxSide;
                 e = fused_forward(which, ft, d_planes, args, d_raw, d_out,
                                   (int)k, temperature, cfg, stream);

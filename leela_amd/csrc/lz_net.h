@@ -58,6 +58,10 @@ struct Net {
     // Batches of at most this many 19x19 boards run the layered form of
     // the 16-bit kernels (fused_forward_layered); 0 disables it.
     int layered_max = kLayeredMaxBoards;
+    // By default also policy batches of up to this many boards, and that many
+    // past whole passes of the chip (see run_net); 0 once a caller has set
+    // a limit of its own.
+    int layered_tail = kLayeredTailBoards;
     int cus = 0;            // compute units of the device
     int occ[3] = {0, 0, 0}; // resident workgroups per CU for wm = 1, 2
     // Launch shape per batch bucket (<=64, <=256, <=1024, more), set by

@@ -13,14 +13,27 @@ from leela_amd.positions import make_batch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def be(weights_a):
+def _backend(weights):
     import leela_amd
     b = leela_amd.Backend(0)
-    pol, val = weights_a
+    pol, val = weights
     b.load_net(leela_amd.NET_POLICY, pol)
     b.load_net(leela_amd.NET_VALUE, val)
     b.finalize()
+    return b
+
+
+@pytest.fixture(scope="module")
+def be(weights_a):
+    b = _backend(weights_a)
+    yield b
+    b.close()
+
+
+@pytest.fixture(scope="module")
+def be_default(weights_a):
+    """A backend whose layered limit is never set."""
+    b = _backend(weights_a)
     yield b
     b.close()
 
@@ -61,7 +74,7 @@ def test_layered_equals_fused_where_bands_split(be, n):
 
 
 @pytest.mark.parametrize("n", [65, 96, 97, 256, 257, 352, 353, 513, 600])
-def test_rest_of_a_policy_batch_equals_fused(be, n):
+def test_rest_of_a_policy_batch_equals_fused(be, be_default, n):
     """Policy batches of up to 96 boards, and up to 96 boards past whole
     passes of 256, run in the layered form: the same bits as the persistent
     kernel's alone, in every row and not past them; also without a raw
@@ -72,21 +85,51 @@ def test_rest_of_a_policy_batch_equals_fused(be, n):
     print(f"case: n={n}", flush=True)
     planes = torch.from_numpy(make_batch(n, seed0=5000 + n)).cuda()
     got = {}
-    for lm in (0, 64):
-        be.set_layered_max(lm)
+    be.set_layered_max(0)
+    for lm, b in ((0, be), (64, be_default)):
         raw = torch.full((n + 1, 361), -7.0, device="cuda")
         out = torch.full((n + 1, 361), -7.0, device="cuda")
         only = torch.full((n + 1, 361), -7.0, device="cuda")
         st = torch.cuda.current_stream().cuda_stream
-        be.forward_device(0, p, n, planes.data_ptr(), raw.data_ptr(),
-                          out.data_ptr(), st)
-        be.forward_device(0, p, n, planes.data_ptr(), None, only.data_ptr(),
-                          st)
+        b.forward_device(0, p, n, planes.data_ptr(), raw.data_ptr(),
+                         out.data_ptr(), st)
+        b.forward_device(0, p, n, planes.data_ptr(), None, only.data_ptr(),
+                         st)
         got[lm] = [t.cpu().numpy() for t in (raw, out, only)]
     be.set_layered_max(64)
     for a, b in zip(got[0], got[64]):
         np.testing.assert_array_equal(a, b)
         assert (b[n] == -7.0).all()
+
+
+@pytest.mark.parametrize("n,limit", [(80, 64), (272, 16), (272, 64)])
+def test_a_limit_that_is_set_holds(be, be_default, n, limit):
+    """Policy batches past a limit that the caller has set run in the
+    persistent kernel as a whole, as they do with the limit 0; the default
+    takes the 80 boards, or the 16 past a pass, in the layered form (0.8 of
+    the time)."""
+    import torch
+    import leela_amd
+    print(f"case: n={n} limit={limit}", flush=True)
+    planes = torch.from_numpy(make_batch(n, seed0=3)).cuda()
+    raw = torch.empty((n, 361), device="cuda")
+    out = torch.empty_like(raw)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def ms(b):
+        return min(float(np.sum(b.forward_timed(
+            0, leela_amd.PREC_FP16, n, planes.data_ptr(), raw.data_ptr(),
+            out.data_ptr(), st))) for _ in range(20))
+
+    be.set_layered_max(0)
+    persistent = ms(be)
+    be.set_layered_max(limit)
+    limited = ms(be)
+    be.set_layered_max(64)
+    default = ms(be_default)
+    print(f"ms: {persistent:.4f} {limited:.4f} {default:.4f}", flush=True)
+    assert abs(limited / persistent - 1) < 0.08
+    assert default < 0.92 * persistent
 
 
 def test_layered_queue_bucket_equals_direct(be):
