@@ -396,21 +396,22 @@ __global__ __launch_bounds__(kFcThreads) void value_fc_kernel(
     float *__restrict__ out, int n, int P, int H,
     const int *__restrict__ n_dev) {
     constexpr int W = kFcThreads / 64;
-    __shared__ f32x4 s_h[kMaxSide * kMaxSide + 8 * W];  // [input] (boards)
+    __shared__ f32x4 s_h[kMaxSide * kMaxSide];  // [input] (boards)
     __shared__ float s_part[W][kFcBoards][256];
     __shared__ float s_red[kFcBoards][W];
     // A replayed graph sizes its grid for the bucket; the batch's board
     // count is then read from device memory.
     if (n_dev) n = min(n, *n_dev);
     const int b0 = blockIdx.x * kFcBoards, tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (b0 >= n) return;
     const int nb = min(kFcBoards, n - b0);
-    for (int i = tid; i < P + 8 * W; i += kFcThreads) {
+    for (int i = tid; i < P; i += kFcThreads) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int bb = 0; bb < kFcBoards; bb++)
-            if (bb < nb && i < P) v[bb] = h0[(size_t)(b0 + bb) * P + i];
+            if (bb < nb) v[bb] = h0[(size_t)(b0 + bb) * P + i];
         s_h[i] = v;
     }
     __syncthreads();
@@ -422,7 +423,8 @@ __global__ __launch_bounds__(kFcThreads) void value_fc_kernel(
         f32x4 acc[kFcBoards];
 #pragma unroll
         for (int bb = 0; bb < kFcBoards; bb++) acc[bb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // Row i0 + u W of W1 (past the last input: the last row, times zeros).
+        // Row i0 + u W of W1 (past the last input the last row, not used: its
+        // weights times zeros would be NaN where one is infinite).
         f32x4 wv[8];
         auto row_at = [&](int i) {
             const float *row = w1t + (size_t)min(i, P - 1) * H;
@@ -437,17 +439,24 @@ __global__ __launch_bounds__(kFcThreads) void value_fc_kernel(
         };
 #pragma unroll
         for (int u = 0; u < 8; u++) wv[u] = row_at(wave + u * W);
-        for (int i0 = wave; i0 < P; i0 += 8 * W) {
+        auto add = [&](const f32x4 &w, const f32x4 &h) {
+#pragma unroll
+            for (int bb = 0; bb < kFcBoards; bb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[bb][r] += w[r] * h[bb];
+        };
+        int i0 = wave;
+        for (; i0 + 7 * W < P; i0 += 8 * W) {
 #pragma unroll
             for (int u = 0; u < 8; u++) {
                 const f32x4 h = s_h[i0 + u * W], w = wv[u];
                 wv[u] = row_at(i0 + (u + 8) * W);
-#pragma unroll
-                for (int bb = 0; bb < kFcBoards; bb++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[bb][r] += w[r] * h[bb];
+                add(w, h);
             }
         }
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (i0 + u * W < P) add(wv[u], s_h[i0 + u * W]);
         __syncthreads();
 #pragma unroll
         for (int bb = 0; bb < kFcBoards; bb++)

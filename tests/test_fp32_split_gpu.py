@@ -112,3 +112,34 @@ def test_value_head_matches_fp64(hidden, n):
     bar = 3e-5 * max(1.0, np.abs(raw64).max())
     assert np.abs(raw.ravel() - raw64.ravel()).max() < bar
     assert np.abs(out.ravel() - out64.ravel()).max() < bar
+
+
+@pytest.mark.parametrize("hidden", [64, 258])
+def test_infinite_value_head_weights(hidden):
+    """An infinite weight of the last input of the first inner product makes
+    its unit infinite, and the value 0, 1 or NaN as in FP32."""
+    import leela_amd
+    from leela_amd import nets
+    print(f"case: hidden={hidden}", flush=True)
+    rng = np.random.default_rng(2)
+    w1 = np.abs(rng.normal(0, 0.1, (hidden, 361))).astype(np.float32)
+    w1[5, 360] = np.inf
+    w2 = rng.normal(0, 0.1, (1, hidden)).astype(np.float32)
+    head = rng.normal(0, 0.1, (1, 4, 3, 3)).astype(np.float32)
+    val = [(nets.CONV, 3, 32, 4, rng.normal(0, 0.1, (4, 32, 3, 3)).astype(
+                np.float32), np.zeros(4, np.float32)),
+           (nets.CONV, 3, 4, 1, head, np.full(1, 0.5, np.float32)),
+           (nets.FC, 0, 361, hidden, w1, np.zeros(hidden, np.float32)),
+           (nets.FC, 0, hidden, 1, w2, np.zeros(1, np.float32))]
+    planes = np.zeros((5, 32, 361), np.uint8)
+    be = leela_amd.Backend(0)
+    try:
+        be.load_net(leela_amd.NET_POLICY, nets.weight_set("A")[0])
+        be.load_net(leela_amd.NET_VALUE, val)
+        be.finalize()
+        raw, _ = be.forward(leela_amd.NET_VALUE, leela_amd.PREC_FP32, planes)
+    finally:
+        be.close()
+    # Empty planes: h0 is 0.5 everywhere, unit 5 +inf.
+    want = np.inf if w2[0, 5] > 0 else -np.inf
+    np.testing.assert_array_equal(raw.ravel(), np.full(5, want, np.float32))
