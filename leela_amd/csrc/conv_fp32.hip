@@ -45,7 +45,8 @@ __device__ __forceinline__ float activate(float v, int act) {
 }
 
 // The three BF16 parts of eight FP32 values. (Values past BF16's largest,
-// 3.39e38, take that as their first part; infinities end up NaN.)
+// 3.39e38, take that as their first part. The third part of an infinity is
+// NaN, and so is every sum that it is in: see conv_split.)
 __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
     constexpr float kMax = 3.3895313892515355e38f;
 #pragma unroll
@@ -66,6 +67,11 @@ __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
 // and halo are split and staged in LDS, HWC, the parts of a pixel side by
 // side (NB = 3 parts of 32 channels; byte planes are exact in one, NB = 1),
 // then F * F k-steps follow. Weights: [chunk][tap][part][m-tile][lane][8].
+//
+// A wave with a sum that is not finite forms its sums again in FP32 (the
+// matrix unit's 16x16x4): the partial products of an infinity, or of a
+// product past FP32's range, have both signs and add up to NaN where FP32 has
+// an infinity. Nothing finite is ever formed twice.
 //
 // Bound: the matrix cores, six products a term. The order of the products
 // gives every operand's reload a group of MFMAs or more before its next
@@ -236,6 +242,71 @@ __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
         }
     }
 
+    float probe = 0.f;  // NaN if any sum is not finite
+#pragma unroll
+    for (int m = 0; m < MTW; m++)
+#pragma unroll
+        for (int t = 0; t < NTW; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                probe = fmaf(acc[m][t][r], 0.f, probe);
+    if (__builtin_amdgcn_ballot_w64(probe != probe)) {
+#pragma unroll
+        for (int m = 0; m < MTW; m++)
+#pragma unroll
+            for (int t = 0; t < NTW; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const __bf16 *wp = (const __bf16 *)wpk;
+        // (The empty asm keeps what is formed here out of the main loop's
+        // registers.)
+        int id = threadIdx.x;
+        asm volatile("" : "+v"(id));
+        const int l = id & 63, w2 = id >> 6;
+        const int m0 = (blockIdx.y * 2 + (w2 & 1)) * MTW;
+#pragma unroll 1
+        for (int k = 0; k < steps * 8; k++) {
+            // Four channels of a tap, one a lane group.
+            const int s = k >> 3, c32 = (k & 7) * 4 + (l >> 4);
+            const int chunk = s / FF, tap = s % FF, c = chunk * 32 + c32;
+            float av[MTW], bv[NTW];
+#pragma unroll
+            for (int m = 0; m < MTW; m++) {
+                const int at =
+                    (m0 + m < mtiles ? m0 + m : mtiles - 1) * 64 + (l & 15) +
+                    16 * (c32 >> 3);
+                float v[3];
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+                    v[p] = (float)wp[((size_t)(s * 3 + p) * mtiles * 64 + at) *
+                                         8 + (c32 & 7)];
+                av[m] = v[0] + v[1] + v[2];
+            }
+#pragma unroll
+            for (int t = 0; t < NTW; t++) {
+                // (Columns past the band: any values, never stored.)
+                const int j = ((w2 >> 1) * NTW + t) * 16 + (l & 15);
+                const int y = y0 + j / kS + tap / F - F / 2;
+                const int x = j % kS + tap % F - F / 2;
+                const bool on = y >= 0 && y < kS && x >= 0 && x < kS;
+                bv[t] = 0.f;
+                if (NB == 1) {
+                    if (on && c < cin)
+                        bv[t] = (float)((const uint8_t *)
+                                            in)[((size_t)board * cin + c) * kP +
+                                                y * kS + x];
+                } else if (on) {
+                    bv[t] = ((const float *)in)[((size_t)board * kP + y * kS +
+                                                 x) * (chunks * 32) + c];
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MTW; m++)
+#pragma unroll
+                for (int t = 0; t < NTW; t++)
+                    acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        av[m], bv[t], acc[m][t], 0, 0, 0);
+        }
+    }
+
     // D layout of 16x16 MFMA: lane holds rows 4*(lane/16)+r of column
     // lane%16: four channels of a pixel.
 #pragma unroll
@@ -271,7 +342,8 @@ __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
 // d[tap][p] = sum_c w[tap][c] x[p][c] (split as above, 16 rows of which nine
 // are used), then out[p] = sum_tap d[tap][p shifted by the tap]. Every input
 // value is read once, straight into an operand. Weights: [chunk][part]
-// [lane][8], lane = tap + 16 * channel group.
+// [lane][8], lane = tap + 16 * channel group. A board with a sum that is not
+// finite is formed again in FP32 (as in conv_split).
 constexpr int kHeadThreads = 512;
 constexpr int kHeadPix = 368;  // 23 column tiles
 
@@ -282,6 +354,7 @@ __device__ __forceinline__ void head_split(const float *__restrict__ src,
                                            float (*d)[kHeadPix],
                                            float *s_out) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float probe = 0.f;  // NaN if any sum is not finite
     for (int t = wave; t < kHeadPix / 16; t += kHeadThreads / 64) {
         const int p = t * 16 + (lane & 15);
         const f32x4 *x = (const f32x4 *)(src + (size_t)(p < kP ? p : kP - 1) *
@@ -309,18 +382,35 @@ __device__ __forceinline__ void head_split(const float *__restrict__ src,
             acc = Op<__bf16>::mfma(a[0], b[0], acc);
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+        for (int r = 0; r < 4; r++) {
             if ((lane >> 4) * 4 + r < 9) d[(lane >> 4) * 4 + r][p] = acc[r];
+            probe = fmaf(acc[r], 0.f, probe);
+        }
     }
-    __syncthreads();
+    const bool again = __syncthreads_or(probe != probe);
     for (int p = tid; p < kP; p += kHeadThreads) {
         const int y = p / kS, x = p % kS;
         float v = 0.0f;
+        if (again) {
+            const __bf16 *wp = (const __bf16 *)w;
+            for (int c = 0; c < chunks * 32; c++)
+                for (int tap = 0; tap < 9; tap++) {
+                    const __bf16 *at =
+                        wp + ((c / 32) * 192 + tap + 16 * (c % 32 / 8)) * 8 +
+                        c % 8;
+                    const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
+                    const bool on = yy >= 0 && yy < kS && xx >= 0 && xx < kS;
+                    v += ((float)at[0] + (float)at[512] + (float)at[1024]) *
+                         (on ? src[(size_t)(yy * kS + xx) * chunks * 32 + c]
+                             : 0.f);
+                }
+        } else {
 #pragma unroll
-        for (int tap = 0; tap < 9; tap++) {
-            const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-            if (yy >= 0 && yy < kS && xx >= 0 && xx < kS)
-                v += d[tap][yy * kS + xx];
+            for (int tap = 0; tap < 9; tap++) {
+                const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
+                if (yy >= 0 && yy < kS && xx >= 0 && xx < kS)
+                    v += d[tap][yy * kS + xx];
+            }
         }
         s_out[p] = activate(v + bias, act);
     }

@@ -222,13 +222,14 @@ float bf16_to_float(uint16_t h) {
     return f;
 }
 
-// The three BF16 parts of f (split3 in conv_fp32.hip).
+// The three BF16 parts of f (split3 in conv_fp32.hip). They add up to f, also
+// to an infinity, which is carried in the third part.
 void split_bf16(float f, uint16_t part[3]) {
     constexpr float kMax = 3.3895313892515355e38f;
     part[0] = float_to_bf16_rne(std::isnan(f) ? f
                                               : std::min(std::max(f, -kMax), kMax));
     float r = f - bf16_to_float(part[0]);
-    part[1] = float_to_bf16_rne(r);
+    part[1] = std::isinf(f) ? 0 : float_to_bf16_rne(r);
     r -= bf16_to_float(part[1]);
     part[2] = float_to_bf16_rne(r);
 }

@@ -147,7 +147,8 @@ int run_net(const Net &net, int which, int precision, int n,
 std::vector<uint16_t> pack_conv_fragments(const Layer &L, FusedType type);
 
 // The FP32 form's weights: each value as three BF16 parts (round to nearest
-// even; the first part of a value past BF16's range is BF16's largest).
+// even; the first part of a value past BF16's range is BF16's largest; an
+// infinity is the third part of its value). The three add up to the weight.
 // Trunk convs: [chunk of 32 inputs][tap][part][m-tile][lane][8], lane = row
 // + 16 * g holding input channels 8*g .. +7 of the chunk; the 3x3 head conv:
 // [chunk][part][lane][8], the taps as rows. Zero past cin, cout and tap 8.

@@ -114,6 +114,100 @@ def test_value_head_matches_fp64(hidden, n):
     assert np.abs(out.ravel() - out64.ravel()).max() < bar
 
 
+def _conv_f32(x, w, b):
+    """Same-padded conv in FP32, term by term, as a matrix product with zero
+    columns off the board forms it: x [n][cin][19][19]."""
+    n, cin = x.shape[:2]
+    cout, _, f, _ = w.shape
+    h = f // 2
+    xp = np.zeros((n, cin, 19 + 2 * h, 19 + 2 * h), np.float32)
+    xp[:, :, h:h + 19, h:h + 19] = x
+    out = np.zeros((n, cout, 19, 19), np.float32)
+    for c in range(cin):
+        for dy in range(f):
+            for dx in range(f):
+                out += (w[:, c, dy, dx][None, :, None, None] *
+                        xp[:, c, dy:dy + 19, dx:dx + 19][:, None])
+    return out + b[None, :, None, None]
+
+
+def _same(got, want, what):
+    """Infinities and NaNs where FP32 has them, the rest as above."""
+    for name, f in (("nan", np.isnan), ("+inf", lambda v: v == np.inf),
+                    ("-inf", lambda v: v == -np.inf)):
+        np.testing.assert_array_equal(f(got), f(want), err_msg=what + name)
+    ok = np.isfinite(want)
+    if ok.any():
+        assert np.abs(got[ok] - want[ok]).max() <= (
+            2e-5 * np.abs(want[ok]).max()), what
+
+
+@pytest.mark.parametrize("n", [1, 130])
+@pytest.mark.parametrize("kind", ["activation", "overflow", "weight",
+                                  "head_weight", "nan_weight"])
+@pytest.mark.parametrize("act", [1, 2])
+def test_infinities_are_those_of_float32(n, kind, act):
+    """Sums that overflow, infinite and NaN activations and weights, with ReLU
+    (which turns a NaN into 0) and with no activation of the trunk: every logit
+    is infinite, NaN or finite as in FP32, and the finite ones agree. One point
+    of every board overflows (or one weight does not hold a number), so most
+    of a board stays finite. n = 1 and 130: pieces of five and ten rows."""
+    import leela_amd
+    from leela_amd import caffe_weights as cw
+    from leela_amd import nets
+    print(f"case: {kind} n={n} act={act}", flush=True)
+    rng = np.random.default_rng(5)
+    shapes = [(5, 3, 40), (3, 40, 33), (3, 33, 1)]
+    table = []
+    for f, cin, cout in shapes:
+        w = rng.normal(0, np.sqrt(2 / (cin * f * f)), (cout, cin, f, f))
+        table.append({"kind": "conv", "filter": f, "cin": cin, "cout": cout,
+                      "w": w.astype(np.float32), "bn": None,
+                      "act": act if cout > 1 else 2,
+                      "b": rng.normal(0, 0.1, cout).astype(np.float32)})
+    planes = np.zeros((n, 3, 361), np.uint8)
+    planes[:, 0] = rng.random((n, 361)) < 0.3
+    w0, w1, w2 = (t["w"] for t in table)
+    # Channel 7 answers to plane 2, set at one point, at that point only.
+    w0[:, 2] = 0
+    w0[7] = 0
+    np.abs(w2, out=w2)
+    planes[:, 2, 23] = 255
+    if kind == "activation":
+        w0[7, 2, 2, 2] = 3e38
+        w1[4, 7] = 0  # 0 x inf
+    elif kind == "overflow":
+        # Finite activations whose products are far past FP32's range.
+        w0[7, 2, 2, 2] = 1e36
+        w1[:, 7] *= 1e12
+    elif kind == "weight":
+        w1[3, 7, 0, 2] = np.inf
+        w1[5, 6, 1, 1] = -np.inf
+    elif kind == "head_weight":
+        w2[0, 3, 2, 0] = np.inf
+    else:
+        w1[9, 2, 1, 0] = np.nan
+    be = leela_amd.Backend(0)
+    try:
+        cw.push_layers(be, leela_amd.NET_POLICY, table)
+        be.load_net(leela_amd.NET_VALUE, nets.weight_set("A")[1])
+        be.finalize()
+        be.set_temperature(1.0)
+        raw, _ = be.forward(leela_amd.NET_POLICY, leela_amd.PREC_FP32, planes)
+    finally:
+        be.close()
+    x = planes.reshape(n, 3, 19, 19).astype(np.float32)
+    with np.errstate(all="ignore"):
+        for t in table:
+            x = _conv_f32(x, t["w"], t["b"])
+            if t["act"] == 1:
+                x = np.where(x > 0, x, np.float32(0))
+    want = x.reshape(n, 361)
+    if kind != "nan_weight" or act == 2:
+        assert not np.isfinite(want).all()
+    _same(raw, want, kind)
+
+
 @pytest.mark.parametrize("hidden", [64, 258])
 def test_infinite_value_head_weights(hidden):
     """An infinite weight of the last input of the first inner product makes
