@@ -2,10 +2,13 @@
 //
 // FP32 convolution on the 16-bit matrix cores (conv_split). Every FP32 value
 // is written as the sum of three BF16 values (round to nearest each time:
-// 8 + 8 + 8 bits and their signs hold the 24 bits exactly, down to 2^-126
-// for the smallest part), and a product is the sum of the six partial
-// products above 2^-25 of it, each exact in FP32:
-//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1 + O(2^-25 a b).
+// 8 + 8 + 8 bits and their signs hold the 24 bits exactly from 2^-103 up;
+// below that the smallest part can be a BF16 subnormal, which the matrix unit
+// takes as 0), and a product is
+// the sum of the six largest partial products, each exact in FP32; the two
+// of up to 2^-25 of it each that are left out make 2^-24 at most (random
+// pairs: 2^-24.04, past 2^-25 for one in a thousand):
+//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1 + O(2^-24 a b).
 // Sums are FP32 throughout (v_mfma_f32_16x16x32_bf16 adds 32 products with
 // fewer roundings than an FP32 chain has), activations stay FP32 in memory.
 // Against 64 bits the nets' outputs are no further off than with FP32 MFMA
@@ -60,6 +63,20 @@ __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
     }
 }
 
+// Sums of products with scaled weights: which cannot stand (see conv_split).
+struct SumProbe {
+    uint32_t small = 0xffffffffu;  // least twice the bits of a sum, less 1
+    float bad = 0.f;               // NaN if a sum is not finite
+    __device__ __forceinline__ void scaled(float v) {
+        const uint32_t b = (__float_as_uint(v) << 1) - 1;
+        small = b < small ? b : small;
+    }
+    __device__ __forceinline__ void sum(float v) { bad = fmaf(v, 0.f, bad); }
+    __device__ __forceinline__ bool again() const {
+        return bad != bad || small < (47u << 24) - 1;  // 0 < |v| < 2^-80
+    }
+};
+
 // One conv. A workgroup computes a band of R image rows of one board (10
 // rows, NTW = 6, or 5, NTW = 3) for 2 * MTW m-tiles of 16 output channels:
 // its four waves are 2 (channels) x 2 (pixels), each MTW m-tiles x NTW
@@ -68,10 +85,15 @@ __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
 // side (NB = 3 parts of 32 channels; byte planes are exact in one, NB = 1),
 // then F * F k-steps follow. Weights: [chunk][tap][part][m-tile][lane][8].
 //
-// A wave with a sum that is not finite forms its sums again in FP32 (the
-// matrix unit's 16x16x4): the partial products of an infinity, or of a
-// product past FP32's range, have both signs and add up to NaN where FP32 has
-// an infinity. Nothing finite is ever formed twice.
+// Weights are over their output channel's scale. A wave with a sum that is
+// not finite, or below 2^-80 and not 0, forms its sums again in FP32 (the
+// matrix unit's 16x16x4, the plain weights). The partial products of an
+// infinity, or of a product past FP32's range, have both signs and add up to
+// NaN where FP32 has an infinity. And what inputs below 2^-103 lack, 2^-126
+// each, is 2^-111 at most over a sum's terms, less than 2^-24 of any sum from
+// 2^-80 up. (Weights below 2^-103 of their channel's largest lack bits for
+// good; that shows only where inputs make up for 30 orders of magnitude.)
+// Ordinary nets never get there.
 //
 // Bound: the matrix cores, six products a term. The order of the products
 // gives every operand's reload a group of MFMAs or more before its next
@@ -81,6 +103,7 @@ __device__ __forceinline__ void split3(const float (&x)[8], bf16x8 (&p)[3]) {
 template <int F, int NB, int MTW, int NTW>
 __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
     const void *__restrict__ in, const bf16x8 *__restrict__ wpk,
+    const float *__restrict__ wscale, const float *__restrict__ wplain,
     const float *__restrict__ bias, float *__restrict__ out, int cin,
     int chunks, int cout, int cstride, int mtiles, ConvEpilogue epi) {
     constexpr int R = NTW == 6 ? 10 : 5, BANDS = (kS + R - 1) / R;
@@ -242,20 +265,26 @@ __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
         }
     }
 
-    float probe = 0.f;  // NaN if any sum is not finite
+    SumProbe probe;
 #pragma unroll
-    for (int m = 0; m < MTW; m++)
+    for (int m = 0; m < MTW; m++) {
+        const int o = (mt0 + m) * 16 + (lane >> 4) * 4;
+        f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+        if (o < cstride) sc = *(const f32x4 *)(wscale + o);
 #pragma unroll
         for (int t = 0; t < NTW; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                probe = fmaf(acc[m][t][r], 0.f, probe);
-    if (__builtin_amdgcn_ballot_w64(probe != probe)) {
+            for (int r = 0; r < 4; r++) {
+                probe.scaled(acc[m][t][r]);
+                acc[m][t][r] *= sc[r];
+                probe.sum(acc[m][t][r]);
+            }
+    }
+    if (__builtin_amdgcn_ballot_w64(probe.again())) {
 #pragma unroll
         for (int m = 0; m < MTW; m++)
 #pragma unroll
             for (int t = 0; t < NTW; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        const __bf16 *wp = (const __bf16 *)wpk;
         // (The empty asm keeps what is formed here out of the main loop's
         // registers.)
         int id = threadIdx.x;
@@ -273,12 +302,7 @@ __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
                 const int at =
                     (m0 + m < mtiles ? m0 + m : mtiles - 1) * 64 + (l & 15) +
                     16 * (c32 >> 3);
-                float v[3];
-#pragma unroll
-                for (int p = 0; p < 3; p++)
-                    v[p] = (float)wp[((size_t)(s * 3 + p) * mtiles * 64 + at) *
-                                         8 + (c32 & 7)];
-                av[m] = v[0] + v[1] + v[2];
+                av[m] = wplain[((size_t)s * mtiles * 64 + at) * 8 + (c32 & 7)];
             }
 #pragma unroll
             for (int t = 0; t < NTW; t++) {
@@ -342,19 +366,23 @@ __global__ __launch_bounds__(kThreads, MTW * NTW > 3 ? 2 : 3) void conv_split(
 // d[tap][p] = sum_c w[tap][c] x[p][c] (split as above, 16 rows of which nine
 // are used), then out[p] = sum_tap d[tap][p shifted by the tap]. Every input
 // value is read once, straight into an operand. Weights: [chunk][part]
-// [lane][8], lane = tap + 16 * channel group. A board with a sum that is not
-// finite is formed again in FP32 (as in conv_split).
+// [lane][8], lane = tap + 16 * channel group, over the conv's scale. Where a
+// sum is not finite or very small FP32 products take its place, as in
+// conv_split.
 constexpr int kHeadThreads = 512;
 constexpr int kHeadPix = 368;  // 23 column tiles
 
 // The activated conv of one board into s_out[0..361).
 __device__ __forceinline__ void head_split(const float *__restrict__ src,
                                            const bf16x8 *__restrict__ w,
-                                           float bias, int chunks, int act,
+                                           const float *__restrict__ wscale,
+                                           const float *__restrict__ wplain,
+                                           float bias, int cin, int act,
                                            float (*d)[kHeadPix],
                                            float *s_out) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    float probe = 0.f;  // NaN if any sum is not finite
+    const int chunks = (cin + 31) / 32;
+    SumProbe probe;
     for (int t = wave; t < kHeadPix / 16; t += kHeadThreads / 64) {
         const int p = t * 16 + (lane & 15);
         const f32x4 *x = (const f32x4 *)(src + (size_t)(p < kP ? p : kP - 1) *
@@ -384,33 +412,31 @@ __device__ __forceinline__ void head_split(const float *__restrict__ src,
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             if ((lane >> 4) * 4 + r < 9) d[(lane >> 4) * 4 + r][p] = acc[r];
-            probe = fmaf(acc[r], 0.f, probe);
+            probe.scaled(acc[r]);
+            probe.sum(acc[r]);
         }
     }
-    const bool again = __syncthreads_or(probe != probe);
+    const bool again = __syncthreads_or(probe.again());
     for (int p = tid; p < kP; p += kHeadThreads) {
         const int y = p / kS, x = p % kS;
         float v = 0.0f;
-        if (again) {
-            const __bf16 *wp = (const __bf16 *)w;
-            for (int c = 0; c < chunks * 32; c++)
+#pragma unroll
+        for (int tap = 0; tap < 9; tap++) {
+            const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
+            if (yy >= 0 && yy < kS && xx >= 0 && xx < kS)
+                v += d[tap][yy * kS + xx];
+        }
+        v *= wscale[0];
+        if (again || !isfinite(v)) {
+            v = 0.0f;
+            for (int c = 0; c < cin; c++)
                 for (int tap = 0; tap < 9; tap++) {
-                    const __bf16 *at =
-                        wp + ((c / 32) * 192 + tap + 16 * (c % 32 / 8)) * 8 +
-                        c % 8;
                     const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
                     const bool on = yy >= 0 && yy < kS && xx >= 0 && xx < kS;
-                    v += ((float)at[0] + (float)at[512] + (float)at[1024]) *
+                    v += wplain[c * 9 + tap] *
                          (on ? src[(size_t)(yy * kS + xx) * chunks * 32 + c]
                              : 0.f);
                 }
-        } else {
-#pragma unroll
-            for (int tap = 0; tap < 9; tap++) {
-                const int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-                if (yy >= 0 && yy < kS && xx >= 0 && xx < kS)
-                    v += d[tap][yy * kS + xx];
-            }
         }
         s_out[p] = activate(v + bias, act);
     }
@@ -434,14 +460,15 @@ __device__ float block_reduce(float v, bool is_max, float *s_red) {
 
 __global__ __launch_bounds__(kHeadThreads) void policy_head_f32_kernel(
     const float *__restrict__ in, const bf16x8 *__restrict__ w,
+    const float *__restrict__ wscale, const float *__restrict__ wplain,
     const float *__restrict__ b, float *__restrict__ raw,
-    float *__restrict__ out, int chunks, float temperature, int act) {
+    float *__restrict__ out, int cin, float temperature, int act) {
     __shared__ float d[9][kHeadPix];
     __shared__ float s_logit[kP];
     __shared__ float s_red[kHeadThreads / 64];
     const int board = blockIdx.x, p = threadIdx.x;
-    head_split(in + (size_t)board * kP * chunks * 32, w, b[0], chunks, act, d,
-               s_logit);
+    head_split(in + (size_t)board * kP * ((cin + 31) / 32 * 32), w, wscale,
+               wplain, b[0], cin, act, d, s_logit);
     // Network::softmax (Network.cpp:450-469): exp(x/T - max/T) / sum.
     const float v = p < kP ? s_logit[p] : -INFINITY;
     const float alpha = block_reduce(v, true, s_red) / temperature;
@@ -456,13 +483,13 @@ __global__ __launch_bounds__(kHeadThreads) void policy_head_f32_kernel(
 // [n][361] for value_fc_head.
 __global__ __launch_bounds__(kHeadThreads) void value_headconv_f32_kernel(
     const float *__restrict__ in, const bf16x8 *__restrict__ w,
-    const float *__restrict__ b, float *__restrict__ h0, int chunks,
-    int act) {
+    const float *__restrict__ wscale, const float *__restrict__ wplain,
+    const float *__restrict__ b, float *__restrict__ h0, int cin, int act) {
     __shared__ float d[9][kHeadPix];
     __shared__ float s_h0[kP];
     const int board = blockIdx.x, p = threadIdx.x;
-    head_split(in + (size_t)board * kP * chunks * 32, w, b[0], chunks, act, d,
-               s_h0);
+    head_split(in + (size_t)board * kP * ((cin + 31) / 32 * 32), w, wscale,
+               wplain, b[0], cin, act, d, s_h0);
     if (p < kP) h0[(size_t)board * kP + p] = s_h0[p];
 }
 
@@ -579,16 +606,16 @@ __global__ __launch_bounds__(kFcThreads) void value_fc_kernel(
 }
 
 template <int F, int NB, int MTW, int NTW>
-hipError_t launch(const void *in, const uint16_t *wpk, const float *bias,
+hipError_t launch(const void *in, const SplitWeights &w, const float *bias,
                   float *out, int n, int cin, int cout,
                   const ConvEpilogue &epi, hipStream_t stream) {
     constexpr int BANDS = NTW == 6 ? 2 : 4;
     const int mtiles = (cout + 15) / 16;
     const dim3 grid(n * BANDS, (mtiles + 2 * MTW - 1) / (2 * MTW));
     hipLaunchKernelGGL((conv_split<F, NB, MTW, NTW>), grid, dim3(kThreads), 0,
-                       stream, in, reinterpret_cast<const bf16x8 *>(wpk), bias,
-                       out, cin, f32_chunks(cin), cout, f32_stride(cout),
-                       mtiles, epi);
+                       stream, in, reinterpret_cast<const bf16x8 *>(w.parts),
+                       w.scale, w.plain, bias, out, cin, f32_chunks(cin), cout,
+                       f32_stride(cout), mtiles, epi);
     return hipGetLastError();
 }
 
@@ -601,7 +628,7 @@ hipError_t launch(const void *in, const uint16_t *wpk, const float *bias,
 // convs at n = 64 take 458 us with one m-tile and five rows a wave, 564 with
 // four; at n = 256 1339 us with four and ten, 1416 with four and five).
 template <int F, int NB>
-hipError_t launch_conv(const void *in, const uint16_t *wpk, const float *bias,
+hipError_t launch_conv(const void *in, const SplitWeights &w, const float *bias,
                        float *out, int n, int cin, int cout,
                        const ConvEpilogue &epi, hipStream_t stream) {
     const int mtiles = (cout + 15) / 16;
@@ -623,9 +650,9 @@ hipError_t launch_conv(const void *in, const uint16_t *wpk, const float *bias,
         }
     auto go = [&](auto m) {
         constexpr int M = decltype(m)::value;
-        return big ? launch<F, NB, M, 6>(in, wpk, bias, out, n, cin, cout, epi,
+        return big ? launch<F, NB, M, 6>(in, w, bias, out, n, cin, cout, epi,
                                          stream)
-                   : launch<F, NB, M, 3>(in, wpk, bias, out, n, cin, cout, epi,
+                   : launch<F, NB, M, 3>(in, w, bias, out, n, cin, cout, epi,
                                          stream);
     };
     switch (mtw) {
@@ -643,42 +670,43 @@ bool act_ok(int act) {
 }  // namespace
 
 hipError_t conv_f32(int filter, bool u8_input, const void *in,
-                    const uint16_t *wpk, const float *bias, float *out, int n,
-                    int cin, int cout, const ConvEpilogue &epi,
+                    const SplitWeights &w, const float *bias, float *out,
+                    int n, int cin, int cout, const ConvEpilogue &epi,
                     hipStream_t stream) {
     if (n <= 0 || cin < 1 || cout < 1 || !act_ok(epi.act) ||
         (epi.bn_mean && !epi.bn_inv_std))
         return hipErrorInvalidValue;
     if (filter == 3)
-        return u8_input ? launch_conv<3, 1>(in, wpk, bias, out, n, cin, cout,
+        return u8_input ? launch_conv<3, 1>(in, w, bias, out, n, cin, cout,
                                             epi, stream)
-                        : launch_conv<3, 3>(in, wpk, bias, out, n, cin, cout,
+                        : launch_conv<3, 3>(in, w, bias, out, n, cin, cout,
                                             epi, stream);
     if (filter == 5)
-        return u8_input ? launch_conv<5, 1>(in, wpk, bias, out, n, cin, cout,
+        return u8_input ? launch_conv<5, 1>(in, w, bias, out, n, cin, cout,
                                             epi, stream)
-                        : launch_conv<5, 3>(in, wpk, bias, out, n, cin, cout,
+                        : launch_conv<5, 3>(in, w, bias, out, n, cin, cout,
                                             epi, stream);
     return hipErrorInvalidValue;
 }
 
-hipError_t policy_head_f32(const float *in, const uint16_t *w, const float *b,
-                           float *raw, float *out, int n, int cin,
-                           float temperature, int act, hipStream_t stream) {
+hipError_t policy_head_f32(const float *in, const SplitWeights &w,
+                           const float *b, float *raw, float *out, int n,
+                           int cin, float temperature, int act,
+                           hipStream_t stream) {
     if (n <= 0 || cin < 1 || !act_ok(act)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(policy_head_f32_kernel, dim3(n), dim3(kHeadThreads), 0,
-                       stream, in, reinterpret_cast<const bf16x8 *>(w), b, raw,
-                       out, f32_chunks(cin), temperature, act);
+                       stream, in, reinterpret_cast<const bf16x8 *>(w.parts),
+                       w.scale, w.plain, b, raw, out, cin, temperature, act);
     return hipGetLastError();
 }
 
-hipError_t value_headconv_f32(const float *in, const uint16_t *w,
+hipError_t value_headconv_f32(const float *in, const SplitWeights &w,
                               const float *b, float *h0, int n, int cin,
                               int act, hipStream_t stream) {
     if (n <= 0 || cin < 1 || !act_ok(act)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(value_headconv_f32_kernel, dim3(n), dim3(kHeadThreads),
-                       0, stream, in, reinterpret_cast<const bf16x8 *>(w), b,
-                       h0, f32_chunks(cin), act);
+                       0, stream, in, reinterpret_cast<const bf16x8 *>(w.parts),
+                       w.scale, w.plain, b, h0, cin, act);
     return hipGetLastError();
 }
 

@@ -34,22 +34,33 @@ struct ConvEpilogue {
     const float *bn_inv_std = nullptr;
 };
 
+// A conv's weights: `parts`, the three BF16 parts of each weight over its
+// output channel's `scale` (a power of two, so that the channel's largest
+// weight is 1 .. 2 and the parts of the others hold all their bits down to
+// 2^-103 of it), as MFMA fragments; `plain`, the FP32 weights themselves.
+// Trunk convs: parts [chunk][tap][part][m-tile][lane][8], plain
+// [chunk][tap][m-tile][lane][8], scale [f32_stride(cout)]. The 3x3 head
+// conv: parts [chunk][part][lane][8], plain [cin][9], scale [1].
+struct SplitWeights {
+    const uint16_t *parts;
+    const float *scale, *plain;
+};
+
 // One same-padded conv over n 19x19 boards. in: byte planes [n][cin][361]
-// (u8_input) or activations; wpk: the three BF16 parts of the weights as MFMA
-// fragments, [chunk][tap][part][m-tile][lane][8].
+// (u8_input) or activations.
 hipError_t conv_f32(int filter, bool u8_input, const void *in,
-                    const uint16_t *wpk, const float *bias, float *out, int n,
-                    int cin, int cout, const ConvEpilogue &epi,
+                    const SplitWeights &w, const float *bias, float *out,
+                    int n, int cin, int cout, const ConvEpilogue &epi,
                     hipStream_t stream);
 
-// Last 1-channel 3x3 conv + activation + softmax(T): raw/out [n][361]. w:
-// the parts of the nine taps' weights, [chunk][part][lane][8].
-hipError_t policy_head_f32(const float *in, const uint16_t *w, const float *b,
-                           float *raw, float *out, int n, int cin,
-                           float temperature, int act, hipStream_t stream);
+// Last 1-channel 3x3 conv + activation + softmax(T): raw/out [n][361].
+hipError_t policy_head_f32(const float *in, const SplitWeights &w,
+                           const float *b, float *raw, float *out, int n,
+                           int cin, float temperature, int act,
+                           hipStream_t stream);
 
 // Last 1-channel conv + activation of the value net into h0 [n][361].
-hipError_t value_headconv_f32(const float *in, const uint16_t *w,
+hipError_t value_headconv_f32(const float *in, const SplitWeights &w,
                               const float *b, float *h0, int n, int cin,
                               int act, hipStream_t stream);
 

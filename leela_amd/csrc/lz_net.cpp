@@ -107,8 +107,11 @@ int upload_net(Net &net, int which, std::string *msg) {
     for (int k = 0; k < (int)net.layers.size() && e == hipSuccess; k++) {
         Layer &L = net.layers[k];
         if (L.kind == Layer::kConv) {
-            e = upload(&L.d_w32,
-                       k < net.head ? pack_conv_split(L) : pack_head_split(L));
+            const SplitPack pk =
+                k < net.head ? pack_conv_split(L) : pack_head_split(L);
+            e = upload(&L.d_w32, pk.parts);
+            if (e == hipSuccess) e = upload(&L.d_wscale, pk.scale);
+            if (e == hipSuccess) e = upload(&L.d_wplain, pk.plain);
         } else if (k == net.fc1) {
             std::vector<float> t(L.w.size());
             for (int o = 0; o < L.cout; o++)
@@ -222,50 +225,72 @@ float bf16_to_float(uint16_t h) {
     return f;
 }
 
-// The three BF16 parts of f (split3 in conv_fp32.hip). They add up to f, also
-// to an infinity, which is carried in the third part.
+// The three BF16 parts of f (split3 in conv_fp32.hip).
 void split_bf16(float f, uint16_t part[3]) {
     constexpr float kMax = 3.3895313892515355e38f;
     part[0] = float_to_bf16_rne(std::isnan(f) ? f
                                               : std::min(std::max(f, -kMax), kMax));
     float r = f - bf16_to_float(part[0]);
-    part[1] = std::isinf(f) ? 0 : float_to_bf16_rne(r);
+    part[1] = float_to_bf16_rne(r);
     r -= bf16_to_float(part[1]);
     part[2] = float_to_bf16_rne(r);
 }
 
-}  // namespace
-
-std::vector<uint16_t> pack_conv_split(const Layer &L) {
-    const int F = L.filter, cin = L.cin, cout = L.cout;
-    const int chunks = f32_chunks(cin), MT = (cout + 15) / 16;
-    std::vector<uint16_t> out((size_t)chunks * F * F * 3 * MT * 512, 0);
-    for (int o = 0; o < cout; o++)
-        for (int c = 0; c < cin; c++)
-            for (int tap = 0; tap < F * F; tap++) {
-                uint16_t part[3];
-                split_bf16(L.w[((size_t)o * cin + c) * F * F + tap], part);
-                const int lane = o % 16 + 16 * (c % 32 / 8);
-                for (int p = 0; p < 3; p++)
-                    out[((((size_t)(c / 32) * F * F + tap) * 3 + p) * MT +
-                         o / 16) * 512 + lane * 8 + c % 8] = part[p];
-            }
-    return out;
+// The exponent of the largest finite magnitude of k weights (0 if they are
+// all zero).
+int top_exponent(const float *w, size_t k) {
+    float top = 0.f;
+    for (size_t i = 0; i < k; i++)
+        if (std::isfinite(w[i])) top = std::max(top, std::fabs(w[i]));
+    return top > 0.f ? std::ilogb(top) : 0;
 }
 
-std::vector<uint16_t> pack_head_split(const Layer &L) {
+}  // namespace
+
+SplitPack pack_conv_split(const Layer &L) {
+    const int F = L.filter, cin = L.cin, cout = L.cout;
+    const int chunks = f32_chunks(cin), MT = (cout + 15) / 16;
+    const size_t row = (size_t)cin * F * F;
+    SplitPack pk;
+    pk.parts.assign((size_t)chunks * F * F * 3 * MT * 512, 0);
+    pk.plain.assign((size_t)chunks * F * F * MT * 512, 0.f);
+    pk.scale.assign(f32_stride(cout), 0.f);
+    for (int o = 0; o < cout; o++) {
+        const int ex = top_exponent(&L.w[o * row], row);
+        pk.scale[o] = std::ldexp(1.f, ex);
+        for (int c = 0; c < cin; c++)
+            for (int tap = 0; tap < F * F; tap++) {
+                const float w = L.w[o * row + (size_t)c * F * F + tap];
+                uint16_t part[3];
+                split_bf16(std::ldexp(w, -ex), part);
+                const size_t step = (size_t)(c / 32) * F * F + tap;
+                const int lane = o % 16 + 16 * (c % 32 / 8);
+                const int at = o / 16 * 512 + lane * 8 + c % 8;
+                for (int p = 0; p < 3; p++)
+                    pk.parts[(step * 3 + p) * MT * 512 + at] = part[p];
+                pk.plain[step * MT * 512 + at] = w;
+            }
+    }
+    return pk;
+}
+
+SplitPack pack_head_split(const Layer &L) {
     const int cin = L.cin;
-    std::vector<uint16_t> out((size_t)f32_chunks(cin) * 3 * 512, 0);
+    const int ex = top_exponent(L.w.data(), L.w.size());
+    SplitPack pk;
+    pk.parts.assign((size_t)f32_chunks(cin) * 3 * 512, 0);
+    pk.plain = L.w;
+    pk.scale.assign(1, std::ldexp(1.f, ex));
     for (int c = 0; c < cin; c++)
         for (int tap = 0; tap < 9; tap++) {
             uint16_t part[3];
-            split_bf16(L.w[(size_t)c * 9 + tap], part);
+            split_bf16(std::ldexp(L.w[(size_t)c * 9 + tap], -ex), part);
             const int lane = tap + 16 * (c % 32 / 8);
             for (int p = 0; p < 3; p++)
-                out[((size_t)(c / 32) * 3 + p) * 512 + lane * 8 + c % 8] =
+                pk.parts[((size_t)(c / 32) * 3 + p) * 512 + lane * 8 + c % 8] =
                     part[p];
         }
-    return out;
+    return pk;
 }
 
 uint16_t float_to_f16_rne(float f) {
@@ -354,6 +379,8 @@ std::vector<uint16_t> pack_conv_fragments(const Layer &L, FusedType type) {
 void free_net(Net &net) {
     for (auto &L : net.layers) {
         dfree(L.d_w32);
+        dfree(L.d_wscale);
+        dfree(L.d_wplain);
         dfree(L.d_fc);
         dfree(L.d_b);
         dfree(L.d_wbf16);
@@ -363,7 +390,7 @@ void free_net(Net &net) {
         dfree(L.d_bn_mean);
         dfree(L.d_bn_inv_std);
         L.d_bn_mean = L.d_bn_inv_std = nullptr;
-        L.d_fc = L.d_b = nullptr;
+        L.d_fc = L.d_b = L.d_wscale = L.d_wplain = nullptr;
         L.d_w32 = nullptr;
         L.d_wbf16 = L.d_wf16 = nullptr;
         L.d_wf8 = nullptr;
@@ -474,22 +501,23 @@ static int run_fp32(const Net &net, int which, int n, const uint8_t *planes,
         epi.act = L.act;
         epi.bn_mean = L.d_bn_mean;
         epi.bn_inv_std = L.d_bn_inv_std;
-        e = conv_f32(L.filter, u8, x, L.d_w32, L.d_b, y, n, L.cin, L.cout, epi,
-                     s);
+        e = conv_f32(L.filter, u8, x, {L.d_w32, L.d_wscale, L.d_wplain}, L.d_b,
+                     y, n, L.cin, L.cout, epi, s);
         if (e == hipSuccess && timer) e = timer->mark(s);
         x = y;
         u8 = false;
     }
     const Layer &H = net.layers[net.head];
     if (e == hipSuccess) {
+        const SplitWeights hw = {H.d_w32, H.d_wscale, H.d_wplain};
         if (which == LZ_NET_POLICY) {
-            e = policy_head_f32(static_cast<const float *>(x), H.d_w32, H.d_b,
-                                raw, out, n, H.cin, temperature, H.act, s);
+            e = policy_head_f32(static_cast<const float *>(x), hw, H.d_b, raw,
+                                out, n, H.cin, temperature, H.act, s);
         } else {
             const Layer &F1 = net.layers[net.fc1];
             const Layer &F2 = net.layers[net.fc2];
-            e = value_headconv_f32(static_cast<const float *>(x), H.d_w32,
-                                   H.d_b, ws.h0, n, H.cin, H.act, s);
+            e = value_headconv_f32(static_cast<const float *>(x), hw, H.d_b,
+                                   ws.h0, n, H.cin, H.act, s);
             if (e == hipSuccess) e = value_fc_head(ws.h0, F1.d_fc, F1.d_b,
                                                    F2.d_fc, F2.d_b, raw, out,
                                                    n, net.side * net.side,

@@ -28,8 +28,9 @@ struct Layer {
     float *d_bn_mean = nullptr;
     float *d_bn_inv_std = nullptr;
     // Device copies.
-    uint16_t *d_w32 = nullptr;  // FP32 form's convs: three BF16 parts
-                                // (pack_conv_split / pack_head_split)
+    uint16_t *d_w32 = nullptr;  // FP32 form's convs (SplitWeights):
+    float *d_wscale = nullptr;  // pack_conv_split / pack_head_split
+    float *d_wplain = nullptr;
     float *d_fc = nullptr;   // FC1 transposed [in][out]; FC2 as is
     float *d_b = nullptr;
     uint16_t *d_wbf16 = nullptr;  // BF16 MFMA fragments (fused kernels)
@@ -146,14 +147,16 @@ int run_net(const Net &net, int which, int precision, int n,
 // 32*cb + 8*g .. +7.
 std::vector<uint16_t> pack_conv_fragments(const Layer &L, FusedType type);
 
-// The FP32 form's weights: each value as three BF16 parts (round to nearest
-// even; the first part of a value past BF16's range is BF16's largest; an
-// infinity is the third part of its value). The three add up to the weight.
-// Trunk convs: [chunk of 32 inputs][tap][part][m-tile][lane][8], lane = row
-// + 16 * g holding input channels 8*g .. +7 of the chunk; the 3x3 head conv:
-// [chunk][part][lane][8], the taps as rows. Zero past cin, cout and tap 8.
-std::vector<uint16_t> pack_conv_split(const Layer &L);
-std::vector<uint16_t> pack_head_split(const Layer &L);
+// The FP32 form's weights (layouts: SplitWeights; chunks of 32 inputs, lane =
+// row + 16 * g holding input channels 8*g .. +7 of the chunk, the head conv's
+// taps as rows): parts rounded to nearest even, an infinity's third one NaN.
+// Zero past cin, cout and tap 8.
+struct SplitPack {
+    std::vector<uint16_t> parts;
+    std::vector<float> scale, plain;
+};
+SplitPack pack_conv_split(const Layer &L);
+SplitPack pack_head_split(const Layer &L);
 
 // OCP e4m3 ("E4M3FN": bias 7, max 448, no infinities) with round to
 // nearest even; magnitudes beyond 448 saturate to 448.

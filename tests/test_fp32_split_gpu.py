@@ -4,15 +4,14 @@ changes: channel counts around its blocks of 16 and chunks of 32, 5x5 and
 3x3 filters first and later, batches that take pieces of ten rows, five rows
 and few channels, byte planes that are not 0 / 1, weights of any scale.
 
-Bar: the parts hold FP32 values exactly and drop less than 2^-25 of a
-product, so a conv errs like an FP32 one: K^(1/2) roundings of 2^-24 on sums
-of K <= 5 * 5 * 160 terms, 4e-6 a layer at worst, six layers at most here:
-2e-5 of the largest logit.
+Bar: the parts hold FP32 values exactly and drop 2^-24 of a product at most
+(see test_dropped_partial_products), and the sums of very small products are
+formed again in FP32, so a conv errs like an FP32 one: K^(1/2) roundings of
+2^-24 on sums of K <= 5 * 5 * 160 terms, 4e-6 a layer at worst, six layers at
+most here: 2e-5 of the largest logit.
 """
 import numpy as np
 import pytest
-
-pytestmark = pytest.mark.gpu
 
 # (filter, cin, cout) of the trunk and head.
 NETS = {
@@ -41,11 +40,46 @@ def _table(name, scale):
     return table
 
 
+def _bf16(x):
+    """Rounded to BF16, to nearest even (finite values)."""
+    u = x.astype(np.float32).view(np.uint32).astype(np.uint64)
+    u = (u + 0x7fff + ((u >> 16) & 1)) & 0xffff0000
+    return u.astype(np.uint32).view(np.float32)
+
+
+def _parts(x):
+    h = _bf16(x)
+    m = _bf16(x - h)
+    return h, m, _bf16(x - h - m)
+
+
+def test_dropped_partial_products():
+    """On the CPU: three parts add up to the value exactly from 2^-103 up,
+    each a BF16 normal number or 0, and six of the nine partial products to
+    the product within 2^-24 of it."""
+    rng = np.random.default_rng(0)
+    x, y = (rng.standard_normal(1 << 20).astype(np.float32) for _ in range(2))
+    x = np.concatenate([x, rng.uniform(1, 2, 1 << 20).astype(np.float32)])
+    y = np.concatenate([y, rng.uniform(1, 2, 1 << 20).astype(np.float32)])
+    for v in (x, np.abs(x) * np.float32(2.0 ** -102) + np.float32(2.0 ** -103)):
+        p = _parts(v)
+        assert (sum(q.astype(np.float64) for q in p) == v).all()
+        assert all(((q == 0) | (np.abs(q) >= 2.0 ** -126)).all() for q in p)
+    a, b = _parts(x), _parts(y)
+    got = sum(a[i].astype(np.float64) * b[j]
+              for i, j in ((0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)))
+    want = x.astype(np.float64) * y
+    assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name,n,scale", [
     ("narrow", 1, 1.0), ("narrow", 67, 1.0), ("odd", 1, 1.0),
     ("odd", 33, 1.0), ("odd", 300, 1.0), ("wide", 2, 1.0), ("wide", 64, 1.0),
     ("wide", 130, 1.0), ("reference_head", 96, 1.0),
-    ("reference_head", 257, 1.0), ("odd", 3, 1e30), ("odd", 3, 1e-25)])
+    ("reference_head", 257, 1.0), ("odd", 3, 1e30), ("odd", 3, 1e-25),
+    ("odd", 3, 1e-33), ("reference_head", 130, 1e-35), ("odd", 3, 1e-37),
+    ("reference_head", 3, 1e-37)])
 def test_fp32_form_matches_fp64(name, n, scale):
     import leela_amd
     import oracle
@@ -73,6 +107,7 @@ def test_fp32_form_matches_fp64(name, n, scale):
         assert np.abs(got - ref).max() < 2e-5 * np.abs(ref).max()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("hidden,n", [(2, 1), (3, 5), (64, 2), (256, 4),
                                       (258, 9), (300, 3), (513, 1)])
 def test_value_head_matches_fp64(hidden, n):
@@ -142,6 +177,7 @@ def _same(got, want, what):
             2e-5 * np.abs(want[ok]).max()), what
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 130])
 @pytest.mark.parametrize("kind", ["activation", "overflow", "weight",
                                   "head_weight", "nan_weight"])
@@ -208,6 +244,7 @@ def test_infinities_are_those_of_float32(n, kind, act):
     _same(raw, want, kind)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("hidden", [64, 258])
 def test_infinite_value_head_weights(hidden):
     """An infinite weight of the last input of the first inner product makes
