@@ -39,7 +39,7 @@ extern "C" {
 #define LZ_NET_VALUE 1
 
 #define LZ_PREC_FP32 0 /* plain form: FP32 everywhere (its products as three-
-                          part BF16 ones on MFMA, exact to 2^-25) */
+                          part BF16 ones on MFMA, within 2^-24 of exact) */
 #define LZ_PREC_BF16 1 /* BF16 trunk on MFMA, FP32 accumulate/epilogue */
 #define LZ_PREC_FP8 2  /* FP8 e4m3 operands after the 5x5 stem (FP16):
                           per-output-channel weight scales, per-board
