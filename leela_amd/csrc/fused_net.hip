@@ -700,14 +700,18 @@ hipError_t launch(int which, int wm, const uint8_t *planes,
 // bit.
 constexpr int kLS = 19;
 constexpr int kLMT = 2;  // output m-tiles per workgroup
-// A prefetch distance of the layered kernels, in k-steps. Measured at 1 / 16
-// / 64 boards (policy, FP16) with one workgroup a band: 2 steps 97 / 113 /
-// 155 us per forward; 1, 3, 4 and 6 steps 118-122 / 141 / 186 (the value net
-// 93 / 100 / 117 for every distance). With two a band, which leave room for
-// it, 8 steps 72.6 / 84.9 against 2 steps 80.5 / 103 (1 / 16 boards).
+// A prefetch distance of the layered stems and head convs, in k-steps (1, 2
+// and 4 steps take the same time within 0.5 us).
 constexpr int kLayeredPF = 2;
 // Most boards whose trunk convs take two workgroups a band.
 constexpr int kSplitPolicy = 25, kSplitValue = 16;
+// A prefetch distance of the trunk convs, in k-steps, with one workgroup a
+// band and with two, which leave room for more. Policy net, FP16, us per
+// forward: one a band 2 steps 86 / 115 / 152 at 1 / 16 / 64 boards, 4 steps
+// 101 / 139 / 179; two a band 8 steps 72 / 84 at 1 / 16 boards, 2 steps 80 /
+// 93. Value net: two a band 4 steps 59.5 / 65, 2 steps 62 / 67.5; one a band
+// the same with 2 and 4.
+constexpr int kTrunkPF = 2, kSplitPolicyPF = 8, kSplitValuePF = 4;
 template <int PS>
 constexpr int lrp() { return (kLS + 2) * PS + row_pad(PS, 2); }
 constexpr int lrp_in() { return (kLS + 4) * kInPS + row_pad(kInPS, 4); }
@@ -1041,12 +1045,15 @@ hipError_t layered_run(int which, const uint8_t *planes, const FusedArgs &a,
         hipLaunchKernelGGL((layered_stem<T, 144, 96>), dim3(n * 3), blk, 0, s,
                            planes, bits, a.w[0], a.b[0], buf[0], n, cnt);
         // Two workgroups a band while that is at most one a CU: policy net
-        // 108 -> 73 us at 1 board, 113 -> 85 at 16; at 32 boards 126 -> 128.
+        // 86 -> 72 us at 1 board, 115 -> 84 at 16, 124 -> 97 at 25; at 32
+        // boards 127 -> 129.
         const int cs = n <= kSplitPolicy ? 2 : 1;
-        const auto first = cs == 2 ? layered_conv<T, 144, 96, 128, 2, kWN, 8>
-                                   : layered_conv<T, 144, 96, 128, 1, kWN, 2>;
-        const auto conv = cs == 2 ? layered_conv<T, 144, 128, 128, 2, kWN, 8>
-                                  : layered_conv<T, 144, 128, 128, 1, kWN, 2>;
+        const auto first =
+            cs == 2 ? layered_conv<T, 144, 96, 128, 2, kWN, kSplitPolicyPF>
+                    : layered_conv<T, 144, 96, 128, 1, kWN, kTrunkPF>;
+        const auto conv =
+            cs == 2 ? layered_conv<T, 144, 128, 128, 2, kWN, kSplitPolicyPF>
+                    : layered_conv<T, 144, 128, 128, 1, kWN, kTrunkPF>;
         const dim3 grid(n * kBands * cs);
         hipLaunchKernelGGL(first, grid, blk, 0, s, buf[0], a.w[1], a.b[1],
                            buf[1], n, cnt);
@@ -1062,11 +1069,12 @@ hipError_t layered_run(int which, const uint8_t *planes, const FusedArgs &a,
         return hipErrorInvalidValue;  // (h0: the value head planes)
     hipLaunchKernelGGL((layered_stem<T, 80, 64>), dim3(n * 2), blk, 0, s,
                        planes, bits, a.w[0], a.b[0], buf[0], n, cnt);
-    // (As above, with two waves each: value net 64.5 -> 60.5 us at 1 board, 68
-    // -> 66 at 16; at 32 boards 70 -> 80.)
+    // (As above, with two waves each: value net 63 -> 59.5 us at 1 board, 67.5
+    // -> 65 at 16; at 25 boards 68 -> 70, at 32 70 -> 79.)
     const int cs = n <= kSplitValue ? 2 : 1;
-    const auto conv = cs == 2 ? layered_conv<T, 80, 64, 64, 2, 2, 4>
-                              : layered_conv<T, 80, 64, 64, 1, kWN, 2>;
+    const auto conv = cs == 2
+                          ? layered_conv<T, 80, 64, 64, 2, 2, kSplitValuePF>
+                          : layered_conv<T, 80, 64, 64, 1, kWN, kTrunkPF>;
     for (int l = 1; l <= 10; l++)
         hipLaunchKernelGGL(conv, dim3(n * kBands * cs), dim3(kWN * 64 / cs), 0,
                            s, buf[(l + 1) & 1], a.w[l], a.b[l], buf[l & 1], n,
