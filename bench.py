@@ -509,8 +509,9 @@ def main() -> int:
     pdenc.playouts_into(po_pos, po_k, 5, d_po.data_ptr(), stream)
     torch.cuda.synchronize(dev)
     gpu_po_s = po_n * po_k / (time.perf_counter() - t0)
-    # The reference's pattern policy on the device (one playout per thread;
-    # the first call uploads its tables and allocates the playout states).
+    # The reference's pattern policy on the device (one playout per
+    # wavefront; the first call uploads its tables and allocates the long
+    # candidate lists).
     d_pw = torch.empty(po_n, dtype=torch.float32, device=dev)
     pdenc.playouts_into(po_pos, 4, 6, d_pw.data_ptr(), stream,
                         positions.PLAYOUT_PATTERN)

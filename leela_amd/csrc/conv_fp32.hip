@@ -15,7 +15,7 @@
 // (policy probabilities of 96 boards 3.7e-6 against 5.1e-6, a trained net's
 // logits 3.7e-6 against 4.2e-6). The FP32 matrix unit runs at 1/16 of the
 // BF16 rate, so six products are 2.7 times its peak: 1024 boards through
-// the policy net take 5.06 ms (243 TFLOP/s of FP32 products), against 15.9
+// the policy net take 5.12 ms (240 TFLOP/s of FP32 products), against 15.9
 // on FP32 MFMA (77 TFLOP/s of 157).
 //
 // The product is the one that the reference forms with im2col + sgemm

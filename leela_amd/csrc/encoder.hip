@@ -823,10 +823,12 @@ hipError_t launch_encode(const EncRecord *d_rec, int n, int symmetry,
     if (!d_ovf) return hipErrorInvalidValue;
     // Up to 1024 boards in four parts: a launch lasts as long as its slowest
     // wavefront, whose ladder readings take turns where they part, and the
-    // chip holds 2048 of these wavefronts. One part against four, us: 111 /
-    // 70 at 1 board, 266 / 148 at 16, 394 / 298 at 256, 525 / 485 at 1024;
-    // at 2048 536 / 564 and at 4096 748 / 914, where the parts' own string
-    // finding only adds to a full chip.
+    // chip holds 2048 of these wavefronts. One part against four, us a call:
+    // 108 / 69 at 1 board, 265 / 149 at 16, 380 / 291 at 256, 506 / 476 at
+    // 1024 (the mean of 18 calls on three sets of positions; the gain at 1024
+    // is 3 to 20% from set to set and box to box); at 2048 517 / 559 and at
+    // 4096 735 / 900, where the parts' own string finding only adds to a full
+    // chip.
     const int parts = n <= 1024 ? 4 : 1;
     hipLaunchKernelGGL(encode_kernel, dim3((n + 7) / 8 * 8 * parts), dim3(64),
                        0, stream, d_rec, n, parts, symmetry, d_policy, d_value,

@@ -593,13 +593,14 @@ int run_net(const Net &net, int which, int precision, int n,
                 !ragged && ws.tiles &&
                 reinterpret_cast<uintptr_t>(d_planes) % 16 == 0;
             // The persistent policy kernel takes a pass of the chip (a board
-            // per CU) as long for a few boards as for all: 205 us up to 200
-            // boards, 190 more for any second pass. The layered form takes
-            // 155 us for 64 and 172 for 96, so batches of that size, and the
-            // boards past whole passes of larger ones, run in it (same
-            // bits): 257 boards 426 -> 335 us, 331 435 -> 399, 352 439 ->
-            // 417, 600 680 -> 653. The value net's passes are of 512 boards
-            // and 95 us: no gain past 64.
+            // per CU) nearly as long for a few boards as for all: 196 us for
+            // 64 boards, 238 for 200, 464 for 257. So batches of up to 96
+            // boards, and the boards past whole passes of larger ones, run
+            // in the layered form (same bits): 64 boards 196 -> 154 us, 96
+            // 197 -> 185, 257 464 -> 350, 331 469 -> 440, 352 472 -> 465, 600
+            // 749 -> 737 (one box; another, of a higher clock under load,
+            // 257 426 -> 335, 352 439 -> 417). The value net's passes are of
+            // 512 boards and 95 us: no gain past 64.
             const int tail = which == 0 && !counts && !bits
                                  ? net.layered_tail
                                  : 0;

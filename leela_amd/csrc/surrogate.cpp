@@ -8,8 +8,9 @@
 //   activations                        13 x B x 361 x 64 BF16 (all kept)
 //   conv-gradient maps                 13 x min(B, 1024) x 361 x 64 BF16
 //   head saves s/f/t                   B x (361 + 64 + 1) FP32
-//   partial sums                       weight gradients of up to 39 chunks of
-//                                      boards, head gradients per board
+//   partial sums                       weight gradients of up to 19 chunks of
+//                                      boards (two partials each), head
+//                                      gradients per board
 #include <cmath>
 #include <cstdio>
 #include <cstring>

@@ -145,10 +145,10 @@ def test_gradients_match_oracle(sur):
 @pytest.mark.parametrize("k", [1, 10, 19, 25, 129, 1025])
 def test_gradient_of_a_batch_is_the_mean_of_its_halves(k):
     """2k boards against their two halves: the factor 1 / n halves exactly, so
-    every gradient map is the half's to the bit, and the weight gradients
-    differ by the order of FP32 sums only (runs of boards per workgroup, the
-    tail of the last run, and the split of the backward pass at 1024
-    boards). Sums of N = 361 n products by magnitude up to 2k boards:
+    every gradient map is half of the half batch's to the bit (in both wave
+    grids of the backward pass, and across its split at 1024 boards), and the
+    weight gradients differ by the order of FP32 sums only (runs of boards per
+    workgroup, the tail of the last run, and the split). Sums of N = 361 n products by magnitude up to 2k boards:
     N^(1/2) ulps at random, 2^-24 * sqrt(361 * 2050) = 5e-5 of the largest
     sum, taken as 1e-4 of the tensor's maximum."""
     print(f"surrogate gradient: 2 x {k} positions", flush=True)
@@ -158,12 +158,23 @@ def test_gradient_of_a_batch_is_the_mean_of_its_halves(k):
     try:
         s.set_params(_random_params(7))
         loss, g = s.gradients(planes, y)
-        la, ga = s.gradients(planes[:k], y[:k])
-        lb, gb = s.gradients(planes[k:], y[k:])
         s.keep_maps(True)
         _, g2 = s.gradients(planes, y)
+        layers = (0, 1, 11, 12)
+        maps = [_bf(s.read_map(1, l, 2 * k)) for l in layers]
+        la, ga = s.gradients(planes[:k], y[:k])
+        halves = [[_bf(s.read_map(1, l, k))] for l in layers]
+        lb, gb = s.gradients(planes[k:], y[k:])
+        for l, h in zip(layers, halves):
+            h.append(_bf(s.read_map(1, l, k)))
     finally:
         s.close()
+    for l, m, h in zip(layers, maps, halves):
+        half = np.concatenate(h) / 2
+        # (A half that is a BF16 subnormal is rounded.)
+        normal = np.abs(half) >= 2.0 ** -126
+        assert normal.mean() > 0.9, l
+        np.testing.assert_array_equal(m[normal], half[normal], err_msg=str(l))
     np.testing.assert_array_equal(g, g2)
     assert abs(loss - (la + lb) / 2) <= 1e-5 * abs(loss)
     want = (ga.astype(np.float64) + gb) / 2
