@@ -454,11 +454,16 @@ int ensure_workspace(Workspace &ws, const Net nets[2], int n,
     return ensure_tiles(ws, msg);
 }
 
+hipError_t zero_device(void *p, size_t bytes) {
+    const hipError_t e = hipMemset(p, 0, bytes);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+
 int ensure_tiles(Workspace &ws, std::string *msg) {
     if (ws.tiles) return LZ_OK;
     const size_t bytes = layered_tile_bytes();
     hipError_t e = hipMalloc(&ws.tiles, bytes);
-    if (e == hipSuccess) e = hipMemset(ws.tiles, 0, bytes);
+    if (e == hipSuccess) e = zero_device(ws.tiles, bytes);
     if (e != hipSuccess) {
         if (ws.tiles) (void)hipFree(ws.tiles);
         ws.tiles = nullptr;

@@ -96,6 +96,11 @@ struct Workspace {
     void *tiles = nullptr;   // layered form's activation tiles (zeroed)
 };
 
+// Zeroes device memory and waits for it: a memset of device memory may return
+// before it is done, and the streams that use the memory next (non-blocking
+// ones) are not ordered after the null stream.
+hipError_t zero_device(void *p, size_t bytes);
+
 // Allocates and zeroes ws.tiles if absent (layered_tile_bytes()).
 int ensure_tiles(Workspace &ws, std::string *msg);
 

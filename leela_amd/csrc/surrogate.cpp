@@ -267,9 +267,9 @@ int lz_surrogate_create(lz_surrogate **out, int device, int max_batch,
                     hd + kCh + 1);
     ok = hipMemcpy(s->p, h.data(), L.total * sizeof(float),
                    hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemset(s->m, 0, L.total * sizeof(float)) == hipSuccess &&
-         hipMemset(s->v, 0, L.total * sizeof(float)) == hipSuccess &&
-         hipMemset(s->zeros, 0, 64) == hipSuccess;
+         lz::zero_device(s->m, L.total * sizeof(float)) == hipSuccess &&
+         lz::zero_device(s->v, L.total * sizeof(float)) == hipSuccess &&
+         lz::zero_device(s->zeros, 64) == hipSuccess;
     if (!ok) {
         release(s);
         delete s;
@@ -308,8 +308,8 @@ int lz_surrogate_set_params(lz_surrogate *s, const float *params) {
     const size_t bytes = layout().total * sizeof(float);
     int rc = s->hip(hipStreamSynchronize(s->stream), "sync");
     if (!rc) rc = s->hip(hipMemcpy(s->p, params, bytes, hipMemcpyHostToDevice), "copy");
-    if (!rc) rc = s->hip(hipMemset(s->m, 0, bytes), "memset");
-    if (!rc) rc = s->hip(hipMemset(s->v, 0, bytes), "memset");
+    if (!rc) rc = s->hip(lz::zero_device(s->m, bytes), "memset");
+    if (!rc) rc = s->hip(lz::zero_device(s->v, bytes), "memset");
     s->step = 0;
     s->packed = false;
     return rc;

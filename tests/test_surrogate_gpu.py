@@ -228,6 +228,40 @@ def test_activation_is_the_float32_elu(n):
         s.close()
 
 
+def test_first_step_of_a_fresh_surrogate():
+    """Moments and the weight gradients' zero block are zeroed at creation
+    (the moments again by set_params), and the first step on the caller's
+    stream waits for it: fresh surrogates that get dirty memory make the same
+    first step."""
+    import torch
+    planes = torch.from_numpy(_value_planes(4, 80)).cuda()
+    y = torch.tensor([0.2, 0.9, 0.5, 0.4], device="cuda")
+    got = []
+    for k in range(5):
+        print(f"case: fresh surrogate {k}", flush=True)
+        junk = [torch.full((1 << 24,), float("nan"), device="cuda")
+                for _ in range(6)]
+        torch.cuda.synchronize()
+        del junk
+        torch.cuda.empty_cache()
+        st = torch.cuda.Stream()
+        s = Surrogate(0, max_batch=4, seed=3)
+        try:
+            if k:
+                s.set_params(got[0][0])
+            start = s.params()
+            s.train_step_device(4, planes.data_ptr(), y.data_ptr(), 1e-3,
+                                stream=st.cuda_stream)
+            st.synchronize()
+            got.append((start, s.params()))
+        finally:
+            s.close()
+    for start, after in got[1:]:
+        np.testing.assert_array_equal(start, got[0][0])
+        np.testing.assert_array_equal(after, got[0][1])
+    assert np.isfinite(got[0][1]).all()
+
+
 def _bf(u16):
     """BF16 bit patterns -> float64."""
     return (u16.astype(np.uint32) << 16).view(np.float32).astype(np.float64)

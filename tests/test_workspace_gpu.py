@@ -173,3 +173,48 @@ def test_host_forward_beside_device_forwards(weights_a):
                 assert torch.equal(o, outs[20])
     finally:
         be.close()
+
+
+def _dirty_memory():
+    """Device memory that the next allocations may get is not zero."""
+    import torch
+    junk = [torch.full((1 << 25,), -1, dtype=torch.int32, device="cuda")
+            for _ in range(6)]
+    torch.cuda.synchronize()
+    del junk
+    torch.cuda.empty_cache()
+
+
+def test_first_forward_on_fresh_tiles(weights_a):
+    """A layered forward on the caller's stream right after its tiles were
+    allocated and zeroed (by the forward itself, or by lz_workspace_create):
+    the same as the next one. The fill has to be waited for, since the
+    caller's stream is not ordered after it."""
+    import torch
+    import leela_amd
+    p = leela_amd.PREC_FP16
+    for k in range(4):
+        _dirty_memory()
+        be = leela_amd.Backend(0)
+        for net, w in enumerate(weights_a):
+            be.load_net(net, w)
+        be.finalize()
+        st = torch.cuda.Stream()
+        d = torch.from_numpy(make_batch(16, seed0=k)).cuda()
+        out = torch.empty((4, 16, 361), device="cuda")
+        torch.cuda.synchronize()
+        be.forward_device(0, p, 16, d.data_ptr(), None, out[0].data_ptr(),
+                          st.cuda_stream)
+        be.forward_device(0, p, 16, d.data_ptr(), None, out[1].data_ptr(),
+                          st.cuda_stream)
+        ws = be.workspace(8)
+        for i in (2, 3):
+            be.forward_device_ws(ws, 0, p, 16 if i == 3 else 8, d.data_ptr(),
+                                 None, out[i].data_ptr(), st.cuda_stream)
+        st.synchronize()
+        print(f"case: fresh backend {k}", flush=True)
+        assert torch.equal(out[0], out[1])
+        assert torch.equal(out[2, :8], out[1, :8])
+        assert torch.equal(out[3], out[1])
+        be.free_workspace(ws)
+        be.close()
